@@ -198,6 +198,23 @@ int wm_setrho3d(double *rho, int64_t np, const double *xp, const double *yp,
                 double dz, double xmmin, double ymmin, double zmmin,
                 int64_t *nskipped, void *stream);
 
+/* wm_setrho3d with a workspace of wm_setrho3d_worksize() bytes (256-byte
+ * aligned; 0: this mesh or count takes none, work may be NULL then).
+ * Particles whose neighbours in the arrays are far apart on the mesh are
+ * then ordered by tiles of the mesh before their charge is added, which
+ * for unordered particles takes a fraction of the time.  The same sums in
+ * another order.  work is zero-filled before its first call, belongs to one
+ * mesh size, and is used by one call at a time (each leaves the counters it
+ * starts from at zero again). */
+int64_t wm_setrho3d_worksize(int64_t np, int64_t nx, int64_t ny, int64_t nz);
+int wm_setrho3d_work(double *rho, int64_t np, const double *xp,
+                     const double *yp, const double *zp, double zgrid,
+                     double q, double wght, int64_t nx, int64_t ny,
+                     int64_t nz, double dx, double dy, double dz,
+                     double xmmin, double ymmin, double zmmin,
+                     int64_t *nskipped, void *work, int64_t worksize,
+                     void *stream);
+
 /* Deposit of particles sorted by cell (no reference counterpart as one
  * call; same sums as setrho3d grouped by cell): computes the cell keys,
  * sorts a permutation by key and reduces each cell's charge before adding

@@ -71,6 +71,62 @@ def test_deposit_matches_oracle(device, order):
     assert abs(r.sum() - total) <= 1e-12 * total
 
 
+@pytest.mark.parametrize("mesh", [(NX, NY, NZ), (33, 16, 47), (5, 70, 31), (250, 255, 510)])
+@pytest.mark.parametrize("order", ["random", "cell_ordered", "drifted", "clumped"])
+@pytest.mark.parametrize("n", [262143, 262144, 300001])
+def test_deposit_with_workspace(device, mesh, order, n):
+    """setrho3d with a workspace: boxes, boxes plane by plane and the binned
+    particles, on meshes whose last tiles of 16 cells are full, cut or one
+    cell thin, with particles outside; below 262144 particles there is
+    no workspace.  FP64 sums in another order: 1e-13 of the peak."""
+    from warp_amd import _native as N
+    nx, ny, nz = mesh
+    hi = (-LO[0], -LO[1], 0.08)
+    d = [(hi[k] - LO[k]) / m for k, m in enumerate(mesh)]
+    x, y, z = [v[:n] for v in _beam(n + 5000, 3)]
+    if order != "random":
+        cell = [((v - LO[k]) / d[k]).astype(int) for k, v in enumerate((x, y, z))]
+        p = np.argsort(cell[0] + nx * (cell[1] + ny * cell[2]), kind="stable")
+        x, y, z = x[p], y[p], z[p]
+    if order == "drifted":  # by half a cell, some out of the mesh
+        z = z + 0.5 * d[2]
+    if order == "clumped":  # one cell holds a third of them
+        x[::3], y[::3], z[::3] = x[0], y[0], z[0]
+    x[5], y[n // 2], z[n - 1] = hi[0] + 1., LO[1] - 1., np.nan
+    inside = np.ones(n, bool)
+    for k, v in enumerate((x, y, z)):
+        inside &= (v >= LO[k]) & ((v - LO[k]) * (1. / d[k]) < mesh[k])
+    need = N.lib().wm_setrho3d_worksize(n, *mesh)
+    assert (need > 0) == (n >= 262144)
+    work = torch.zeros(need, dtype=torch.uint8, device=device)
+    keep = [_t(v, device) for v in (x, y, z)]
+    ns = C.c_int64(-1)
+    q, w = 1.602176565e-19, 3.7e12
+    for _ in range(2):  # the first call leaves the workspace as it found it
+        rho = torch.ones((nz + 1, ny + 1, nx + 1), dtype=torch.float64, device=device)
+        N.call("wm_setrho3d_work", rho.data_ptr(), n, *[k.data_ptr() for k in keep], 0.0, q, w,
+               nx, ny, nz, *d, *LO, C.byref(ns), work.data_ptr() if need else None, need,
+               N.stream_of(device))
+        assert ns.value == n - inside.sum()
+    ro = np.ones((nz + 1, ny + 1, nx + 1))
+    O.setrho3d(ro, x[inside], y[inside], z[inside], q, w, *d, *LO)
+    r = rho.cpu().numpy()
+    # n additions of one sign: the oracle's serial sum itself carries up to
+    # the count of a node's particles times half an ulp
+    tol = 1e-13 if order != "clumped" else n / 3 * 1.2e-16
+    assert np.abs(r - ro).max() <= tol * np.abs(ro).max()
+
+
+def test_deposit_worksize_limits():
+    """No workspace for meshes of more tiles than a block can count."""
+    from warp_amd import _native as N
+    f = N.lib().wm_setrho3d_worksize
+    assert f(10 ** 6, 512, 512, 192) > 0       # 32 x 32 x 12 tiles
+    assert f(10 ** 6, 512, 512, 193) == 0
+    assert f(1 << 31, 64, 64, 64) == 0
+    assert f(0, 64, 64, 64) == 0
+
+
 def test_deposit_skips_out_of_grid(device):
     from warp_amd import _native as N
     x = np.array([0.0, 0.03, -0.025, 0.0])

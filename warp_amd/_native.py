@@ -64,6 +64,9 @@ SIGNATURES = {
     "wm_applyboundaryconditions3d": (C.c_int, [_i64, _i64, _i64, _P, _P, _i64, _i64, _P]),
     "wm_setrho3d": (C.c_int, [_P, _i64, _P, _P, _P, _d, _d, _d, _i64, _i64, _i64, _d, _d,
                               _d, _d, _d, _d, _P, _P]),
+    "wm_setrho3d_worksize": (_i64, [_i64, _i64, _i64, _i64]),
+    "wm_setrho3d_work": (C.c_int, [_P, _i64, _P, _P, _P, _d, _d, _d, _i64, _i64, _i64, _d, _d,
+                                   _d, _d, _d, _d, _P, _P, _i64, _P]),
     "wm_setrho3d_sorted_worksize": (_i64, [_i64, _i64, _i64, _i64]),
     "wm_setrho3d_sorted": (C.c_int, [_P, _i64, _P, _P, _P, _d, _d, _d, _i64, _i64, _i64,
                                      _d, _d, _d, _d, _d, _d, _P, _P]),

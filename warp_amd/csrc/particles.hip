@@ -102,20 +102,51 @@ __device__ inline void corner_charges(double u1, double v1, double w1, double g,
 // different nodes instead of piling onto the few nodes of one cell.  The
 // block first finds the box of mesh nodes its particles touch; when it fits
 // in LDS (a few hundred nodes for ordered particles) the charges are summed
-// there and the box is added to rho with one atomic per touched node,
-// otherwise every particle adds its eight charges to rho directly.
-#define DEP_BOX 2048
+// there and the box is added to rho with one atomic per touched node.  A
+// box that does not fit is tried plane by plane of cells, which is what an
+// ordered beam needs at the end of every plane and after it has drifted
+// across a plane of nodes (32M particles ordered by cell on 256x256x512: 416
+// -> 335 us for a uniform beam, 435 -> 392 us for a Gaussian one; 4M on
+// 128x128x256: 147 -> 73 us).  What then remains (unordered particles, or
+// ordered ones so sparse that a block spans many rows) goes on the list of
+// the binned deposit below; without a list (no workspace) every particle
+// adds its eight charges to rho directly, which the rate of global FP64
+// atomics limits to about 17 per ns.
+// DEP_BOX: 3072 nodes (24 KB, six blocks per compute unit) was 2-5% faster
+// than 2048, 4096 and 6144 were slower (435 and 492 us on the Gaussian beam
+// above) for want of resident blocks.
+#define DEP_BOX 3072
 #define DEP_K 4
+#define DEP_PART (256 * DEP_K)
+#define DEP_PLANES 4
+
+// Workspace of the binned deposit (below).
+constexpr int BIN_T = 16;                  // cells per tile and axis
+struct BinWork {
+  unsigned int *head;    // 0: listed blocks (NULL head: no list), 1: pieces
+  unsigned int *count;   // their particles per tile
+  unsigned int *cursor;  // of them brought into tile order so far
+  unsigned int *list;
+  uint3 *piece;          // tile, first, number
+  double *x, *y, *z;     // positions in tile order
+  int ntx, nty, ntiles;
+};
+
+__device__ inline int bin_tile(const BinWork &b, long long ii, long long jj, long long kk) {
+  return (int)ii / BIN_T + b.ntx * ((int)jj / BIN_T + b.nty * ((int)kk / BIN_T));
+}
+
 __global__ __launch_bounds__(256) void k_setrho(double *__restrict__ rho, long long np,
                                                 const double *__restrict__ xp,
                                                 const double *__restrict__ yp,
                                                 const double *__restrict__ zp, Mesh m,
                                                 double g,
-                                                unsigned long long *__restrict__ nskip) {
+                                                unsigned long long *__restrict__ nskip,
+                                                BinWork bin) {
   __shared__ double box[DEP_BOX];
-  __shared__ int lim[4][6];
+  __shared__ int lim[4][6], plim[4][DEP_PLANES][4];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const long long base = (long long)blockIdx.x * 256 * DEP_K + (long long)(l * 4 + w) * DEP_K;
+  const long long base = (long long)blockIdx.x * DEP_PART + (long long)(l * 4 + w) * DEP_K;
   long long ii[DEP_K], jj[DEP_K], kk[DEP_K];
   double u1[DEP_K], v1[DEP_K], w1[DEP_K];
   bool ok[DEP_K];
@@ -156,49 +187,303 @@ __global__ __launch_bounds__(256) void k_setrho(double *__restrict__ rho, long l
   if (a1 < a0) return;  // no particle of the block is in the grid
   const long long sx = m.nx + 1, sxy = (long long)(m.nx + 1) * (m.ny + 1);
   const long long nbx = a1 - a0 + 2, nby = b1 - b0 + 2, nbz = c1 - c0 + 2;
-  if (nbx * nby * nbz > DEP_BOX) {
+  // the charges of the particles in planes p0..p1 (all of them in the box
+  // of nodes of q0 + [0, n)) summed in LDS and added to rho
+  auto sum_box = [&](int p0, int p1, int qx, int qy, int bx, int by) {
+    const int bxy = bx * by, nb = bxy * (p1 - p0 + 2);
+    for (int e = threadIdx.x; e < nb; e += 256) box[e] = 0.;
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < DEP_K; k++) {
-      if (!ok[k]) continue;
+      if (!ok[k] || kk[k] < p0 || kk[k] > p1) continue;
       double c[8];
       corner_charges(u1[k], v1[k], w1[k], g, c);
-      double *r = rho + ii[k] + sx * jj[k] + sxy * kk[k];
-      atomicAdd(r, c[0]);
-      atomicAdd(r + 1, c[1]);
-      atomicAdd(r + sx, c[2]);
-      atomicAdd(r + sx + 1, c[3]);
-      atomicAdd(r + sxy, c[4]);
-      atomicAdd(r + sxy + 1, c[5]);
-      atomicAdd(r + sxy + sx, c[6]);
-      atomicAdd(r + sxy + sx + 1, c[7]);
+      double *bp = box + ((int)ii[k] - qx) + bx * ((int)jj[k] - qy) + bxy * ((int)kk[k] - p0);
+      atomicAdd(bp, c[0]);
+      atomicAdd(bp + 1, c[1]);
+      atomicAdd(bp + bx, c[2]);
+      atomicAdd(bp + bx + 1, c[3]);
+      atomicAdd(bp + bxy, c[4]);
+      atomicAdd(bp + bxy + 1, c[5]);
+      atomicAdd(bp + bxy + bx, c[6]);
+      atomicAdd(bp + bxy + bx + 1, c[7]);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < nb; e += 256) {
+      double v = box[e];
+      if (v != 0.) {
+        int ex = e % bx, ey = e / bx % by, ez = e / bxy;
+        atomicAdd(rho + (qx + ex) + sx * (qy + ey) + sxy * (p0 + ez), v);
+      }
+    }
+  };
+  if (nbx * nby * nbz <= DEP_BOX) {
+    sum_box(c0, c1, a0, b0, (int)nbx, (int)nby);
+    return;
+  }
+  // A block of ordered particles that goes on from one plane of cells to
+  // the next (at the end of a plane, or because a plane's particles have
+  // drifted across a plane of nodes) touches a small box in each of them.
+  int pa[DEP_PLANES][4];
+  bool fits = c1 - c0 < DEP_PLANES;
+  if (fits) {
+#pragma unroll
+    for (int p = 0; p < DEP_PLANES; p++) {
+      int x0 = big, x1 = -big, y0 = big, y1 = -big;
+#pragma unroll
+      for (int k = 0; k < DEP_K; k++)
+        if (ok[k] && kk[k] == c0 + p) {
+          x0 = min(x0, (int)ii[k]);
+          x1 = max(x1, (int)ii[k]);
+          y0 = min(y0, (int)jj[k]);
+          y1 = max(y1, (int)jj[k]);
+        }
+      for (int off = 32; off > 0; off >>= 1) {
+        x0 = min(x0, __shfl_xor(x0, off, 64)); x1 = max(x1, __shfl_xor(x1, off, 64));
+        y0 = min(y0, __shfl_xor(y0, off, 64)); y1 = max(y1, __shfl_xor(y1, off, 64));
+      }
+      if (l == 0) {
+        plim[w][p][0] = x0; plim[w][p][1] = x1; plim[w][p][2] = y0; plim[w][p][3] = y1;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < DEP_PLANES; p++) {
+      for (int q = 0; q < 4; q++) {
+        const int v0 = plim[0][p][q], v1 = plim[1][p][q], v2 = plim[2][p][q], v3 = plim[3][p][q];
+        pa[p][q] = q & 1 ? max(max(v0, v1), max(v2, v3)) : min(min(v0, v1), min(v2, v3));
+      }
+      if (pa[p][1] >= pa[p][0] &&
+          (long long)(pa[p][1] - pa[p][0] + 2) * (pa[p][3] - pa[p][2] + 2) * 2 > DEP_BOX)
+        fits = false;
+    }
+  }
+  if (fits) {
+#pragma unroll
+    for (int p = 0; p < DEP_PLANES; p++) {
+      if (pa[p][1] < pa[p][0]) continue;
+      sum_box(c0 + p, c0 + p, pa[p][0], pa[p][2], pa[p][1] - pa[p][0] + 2,
+              pa[p][3] - pa[p][2] + 2);
+      __syncthreads();
     }
     return;
   }
-  const int bx = (int)nbx, bxy = (int)(nbx * nby), nb = (int)(nbx * nby * nbz);
-  for (int e = threadIdx.x; e < nb; e += 256) box[e] = 0.;
-  __syncthreads();
+  if (bin.head) {
+    // listed, its particles counted per tile: two 16-bit counters a word
+    // (a block has 1024 particles) in the box's memory
+    if (threadIdx.x == 0) bin.list[atomicAdd(bin.head, 1u)] = blockIdx.x;
+    unsigned int *cnt = (unsigned int *)box;
+    for (int t = threadIdx.x; 2 * t < bin.ntiles; t += 256) cnt[t] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < DEP_K; k++)
+      if (ok[k]) {
+        const int t = bin_tile(bin, ii[k], jj[k], kk[k]);
+        atomicAdd(&cnt[t >> 1], 1u << (16 * (t & 1)));
+      }
+    __syncthreads();
+    for (int t = threadIdx.x; 2 * t < bin.ntiles; t += 256) {
+      const unsigned int c = cnt[t];
+      if (c & 0xffffu) atomicAdd(&bin.count[2 * t], c & 0xffffu);
+      if (c >> 16) atomicAdd(&bin.count[2 * t + 1], c >> 16);
+    }
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < DEP_K; k++) {
     if (!ok[k]) continue;
     double c[8];
     corner_charges(u1[k], v1[k], w1[k], g, c);
-    double *bp = box + (ii[k] - a0) + bx * (jj[k] - b0) + bxy * (kk[k] - c0);
-    atomicAdd(bp, c[0]);
-    atomicAdd(bp + 1, c[1]);
-    atomicAdd(bp + bx, c[2]);
-    atomicAdd(bp + bx + 1, c[3]);
-    atomicAdd(bp + bxy, c[4]);
-    atomicAdd(bp + bxy + 1, c[5]);
-    atomicAdd(bp + bxy + bx, c[6]);
-    atomicAdd(bp + bxy + bx + 1, c[7]);
+    double *r = rho + ii[k] + sx * jj[k] + sxy * kk[k];
+    atomicAdd(r, c[0]);
+    atomicAdd(r + 1, c[1]);
+    atomicAdd(r + sx, c[2]);
+    atomicAdd(r + sx + 1, c[3]);
+    atomicAdd(r + sxy, c[4]);
+    atomicAdd(r + sxy + 1, c[5]);
+    atomicAdd(r + sxy + sx, c[6]);
+    atomicAdd(r + sxy + sx + 1, c[7]);
+  }
+}
+
+// The binned deposit of the listed blocks' particles: their positions are
+// brought into the order of tiles of BIN_T^3 cells, and a block then sums a
+// piece of one tile's particles into the tile's (BIN_T+1)^3 nodes in LDS and
+// adds these to rho, so that rho sees one atomic per touched node and piece,
+// in rows of up to BIN_T+1 neighbours, instead of eight scattered ones per
+// particle.  Bound by the two reads and one write of the positions
+// and the LDS atomics: 4M unordered particles on 128x128x256 take 265 us where
+// the scattered atomics took 1910 us, 16M 0.92 ms against 7.6, 32M on
+// 256x256x512 2.4 ms against 10.9.  All sizes come from the device-side list, so
+// the two launches return at once when it is empty (4 us).
+constexpr int BIN_NODES = (BIN_T + 1) * (BIN_T + 1) * (BIN_T + 1);
+constexpr int BIN_MAXTILES = 4 * DEP_BOX;  // 16-bit counters of one k_setrho block
+constexpr int BIN_THREADS = 1024;
+constexpr int BIN_GROUP = 8;               // listed blocks taken at a time at most, one
+                                           // particle of each per thread
+constexpr int BIN_PIECE = 4096;            // particles per piece of a tile, at least
+constexpr int BIN_PIECES = 2048;           // pieces beyond one per tile, at most
+// Fewer particles than this take no workspace: unordered, 100,000 take 54 us
+// by scattered atomics and 27 us binned, 200,000 (on 64^3) 175 and 38 us, but
+// ordered, as a step driver keeps them, they need no list, and the two more
+// launches cost such a short step 1% (5.47 -> 5.53 ms per five steps on 64^3
+// with 200,000).
+constexpr int BIN_MIN = 262144;
+static_assert(DEP_PART == BIN_THREADS, "one particle of a listed block per thread");
+
+// Exclusive sum of v over the block's BIN_THREADS threads; total to all.
+__device__ inline unsigned int bin_scan(unsigned int v, unsigned int *ws, unsigned int &total) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  unsigned int incl = v;
+  for (int off = 1; off < 64; off <<= 1) {
+    const unsigned int o = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += o;
+  }
+  if (lane == 63) ws[wv] = incl;
+  __syncthreads();
+  unsigned int before = 0;
+  total = 0;
+  for (int k = 0; k < BIN_THREADS / 64; k++) {
+    if (k < wv) before += ws[k];
+    total += ws[k];
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < nb; e += 256) {
-    double v = box[e];
-    if (v != 0.) {
-      int ex = e % bx, ey = (e / bx) % (int)nby, ez = e / bxy;
-      atomicAdd(rho + (a0 + ex) + sx * (b0 + ey) + sxy * (c0 + ez), v);
+  return before + incl - v;
+}
+
+// Positions of the listed blocks' particles to tile order.  Every block
+// scans the tiles' counts for itself (a launch of its own for that costs
+// more); block 0 also cuts the tiles into pieces.  A block counts its
+// particles per tile in LDS (the value an atomic returns is the particle's
+// rank), so that a tile's cursor takes one atomic per block and group.
+__global__ __launch_bounds__(BIN_THREADS) void k_bin_scatter(long long np,
+                                                             const double *__restrict__ xp,
+                                                             const double *__restrict__ yp,
+                                                             const double *__restrict__ zp,
+                                                             Mesh m, BinWork b) {
+  extern __shared__ unsigned int lds[];
+  __shared__ unsigned int ws[BIN_THREADS / 64];
+  unsigned int *first = lds, *cnt = lds + b.ntiles;
+  const int n = (int)b.head[0];
+  if (n == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) b.head[1] = 0;
+    return;
+  }
+  const int per = (b.ntiles + BIN_THREADS - 1) / BIN_THREADS;
+  const int t0 = min((int)threadIdx.x * per, b.ntiles), t1 = min(t0 + per, b.ntiles);
+  unsigned int sum = 0, total;
+  for (int t = t0; t < t1; t++) sum += b.count[t];
+  unsigned int at = bin_scan(sum, ws, total);
+  if (blockIdx.x == 0) {
+    const unsigned int size =
+        max((unsigned int)BIN_PIECE, (total + BIN_PIECES - 1) / BIN_PIECES);
+    unsigned int mine = 0, npieces, o = at;
+    for (int t = t0; t < t1; t++) mine += (b.count[t] + size - 1) / size;
+    unsigned int q = bin_scan(mine, ws, npieces);
+    for (int t = t0; t < t1; t++) {
+      const unsigned int c = b.count[t];
+      for (unsigned int d = 0; d < c; d += size)
+        b.piece[q++] = make_uint3((unsigned int)t, o + d, min(size, c - d));
+      o += c;
     }
+    if (threadIdx.x == 0) b.head[1] = npieces;
+  }
+  for (int t = t0; t < t1; t++) {
+    first[t] = at;
+    at += b.count[t];
+  }
+  // listed blocks taken at a time: fewer where there are few
+  const int grp = min(max(n / (int)gridDim.x, 1), BIN_GROUP);
+  for (int g = blockIdx.x * grp; g < n; g += gridDim.x * grp) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < b.ntiles; t += BIN_THREADS) cnt[t] = 0;
+    __syncthreads();
+    double x[BIN_GROUP], y[BIN_GROUP], z[BIN_GROUP];
+    int tile[BIN_GROUP];
+    unsigned int rank[BIN_GROUP];
+#pragma unroll
+    for (int k = 0; k < BIN_GROUP; k++) {
+      const long long ip =
+          k < grp && g + k < n ? (long long)b.list[g + k] * DEP_PART + threadIdx.x : np;
+      tile[k] = -1;
+      if (ip < np) {
+        x[k] = xp[ip];
+        y[k] = yp[ip];
+        z[k] = zp[ip];
+        tile[k] = 0;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < BIN_GROUP; k++) {
+      if (tile[k] < 0) continue;
+      long long ii, jj, kk;
+      double u1, v1, w1;
+      tile[k] = cic(m, x[k], y[k], z[k], ii, jj, kk, u1, v1, w1) ? bin_tile(b, ii, jj, kk) : -1;
+      if (tile[k] >= 0) rank[k] = atomicAdd(&cnt[tile[k]], 1u);
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < b.ntiles; t += BIN_THREADS)
+      if (cnt[t]) cnt[t] = first[t] + atomicAdd(&b.cursor[t], cnt[t]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < BIN_GROUP; k++)
+      if (tile[k] >= 0) {
+        const unsigned int p = cnt[tile[k]] + rank[k];
+        b.x[p] = x[k];
+        b.y[p] = y[k];
+        b.z[p] = z[k];
+      }
+  }
+}
+
+// The pieces; and the counters back to zero for the next deposit (nothing
+// here reads them, and b.head[1] is written anew by every k_bin_scatter).
+__global__ __launch_bounds__(512) void k_bin_deposit(double *__restrict__ rho, Mesh m, double g,
+                                                     BinWork b) {
+  __shared__ double box[BIN_NODES];
+  constexpr int B1 = BIN_T + 1, B2 = B1 * B1;
+  const int np = (int)b.head[1];
+  if (np == 0) {
+    // listed blocks without a particle in the grid are possible: none here
+    // counts, but the list itself starts over
+    if (blockIdx.x == 0 && threadIdx.x == 0) b.head[0] = 0;
+    return;
+  }
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) b.head[0] = 0;
+    for (int t = threadIdx.x; t < b.ntiles; t += 512) b.count[t] = b.cursor[t] = 0;
+  }
+  const long long sx = m.nx + 1, sxy = (long long)(m.nx + 1) * (m.ny + 1);
+  for (int p = blockIdx.x; p < np; p += gridDim.x) {
+    const uint3 pc = b.piece[p];
+    const int t = (int)pc.x;
+    const int i0 = t % b.ntx * BIN_T, j0 = t / b.ntx % b.nty * BIN_T,
+              k0 = t / (b.ntx * b.nty) * BIN_T;
+    for (int e = threadIdx.x; e < BIN_NODES; e += 512) box[e] = 0.;
+    __syncthreads();
+    for (unsigned int q = threadIdx.x; q < pc.z; q += 512) {
+      const long long ip = (long long)pc.y + q;
+      long long ii, jj, kk;
+      double u1, v1, w1, c[8];
+      cic(m, b.x[ip], b.y[ip], b.z[ip], ii, jj, kk, u1, v1, w1);
+      corner_charges(u1, v1, w1, g, c);
+      double *bp = box + ((int)ii - i0) + B1 * ((int)jj - j0) + B2 * ((int)kk - k0);
+      atomicAdd(bp, c[0]);
+      atomicAdd(bp + 1, c[1]);
+      atomicAdd(bp + B1, c[2]);
+      atomicAdd(bp + B1 + 1, c[3]);
+      atomicAdd(bp + B2, c[4]);
+      atomicAdd(bp + B2 + 1, c[5]);
+      atomicAdd(bp + B2 + B1, c[6]);
+      atomicAdd(bp + B2 + B1 + 1, c[7]);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < BIN_NODES; e += 512) {
+      const double v = box[e];
+      if (v != 0.)  // never beyond the mesh: those nodes got no charge
+        atomicAdd(rho + (i0 + e % B1) + sx * (j0 + e / B1 % B1) + sxy * (k0 + e / B2), v);
+    }
+    __syncthreads();
   }
 }
 
@@ -681,6 +966,40 @@ static double deposit_g(double q, double wght, int64_t nx, int64_t ny, int64_t n
   return g;
 }
 
+// Layout of the binned deposit's workspace; total = 0 for few particles,
+// and where the mesh has more tiles than a block counts in LDS or the
+// particle numbers do not fit 32 bits (the deposit then runs without it).
+struct BinLayout {
+  size_t cursor, list, piece, x, y, z, total;
+  int ntx, nty, ntiles;
+};
+
+static BinLayout bin_layout(int64_t np, int64_t nx, int64_t ny, int64_t nz) {
+  BinLayout w{};
+  const int64_t ntx = cdiv(nx, BIN_T), nty = cdiv(ny, BIN_T), ntz = cdiv(nz, BIN_T);
+  if (ntx * nty * ntz > BIN_MAXTILES || np >= (1ll << 31) || np < BIN_MIN) return w;
+  w.ntx = (int)ntx;
+  w.nty = (int)nty;
+  w.ntiles = (int)(ntx * nty * ntz);
+  size_t at = 256;
+  auto take = [&](size_t bytes) {
+    size_t p = at;
+    at += (bytes + 255) & ~(size_t)255;
+    return p;
+  };
+  // the head and the counts first, in a place that depends on the mesh
+  // alone: they are zero between calls
+  take(sizeof(unsigned int) * (size_t)w.ntiles);
+  w.cursor = take(sizeof(unsigned int) * (size_t)w.ntiles);
+  w.list = take(sizeof(unsigned int) * (size_t)cdiv(np, DEP_PART));
+  w.piece = take(sizeof(uint3) * (size_t)(BIN_PIECES + w.ntiles));
+  w.x = take(sizeof(double) * (size_t)np);
+  w.y = take(sizeof(double) * (size_t)np);
+  w.z = take(sizeof(double) * (size_t)np);
+  w.total = at;
+  return w;
+}
+
 struct SortedWork {
   size_t keys, idx, keys2, idx2, temp, total;
 };
@@ -710,16 +1029,23 @@ static int key_bits(int64_t ncell) {
 
 extern "C" {
 
-int wm_setrho3d(double *rho, int64_t np, const double *xp, const double *yp, const double *zp,
-                double zgrid, double q, double wght, int64_t nx, int64_t ny, int64_t nz,
-                double dx, double dy, double dz, double xmmin, double ymmin, double zmmin,
-                int64_t *nskipped, void *stream) {
+int64_t wm_setrho3d_worksize(int64_t np, int64_t nx, int64_t ny, int64_t nz) {
+  return nx > 0 && ny > 0 && nz > 0 ? (int64_t)bin_layout(np, nx, ny, nz).total : 0;
+}
+
+int wm_setrho3d_work(double *rho, int64_t np, const double *xp, const double *yp,
+                     const double *zp, double zgrid, double q, double wght, int64_t nx,
+                     int64_t ny, int64_t nz, double dx, double dy, double dz, double xmmin,
+                     double ymmin, double zmmin, int64_t *nskipped, void *work, int64_t worksize,
+                     void *stream) {
   WM_ENTRY({
     check_grid(nx, ny, nz);
     WM_REQUIRE(np >= 0, "wm_setrho3d: np < 0");
     if (nskipped) *nskipped = 0;
     if (np == 0) return 0;
     WM_REQUIRE(rho && xp && yp && zp, "wm_setrho3d: NULL array");
+    const BinLayout w = work ? bin_layout(np, nx, ny, nz) : BinLayout{};
+    WM_REQUIRE(!w.total || worksize >= (int64_t)w.total, "wm_setrho3d: workspace too small");
     hipStream_t s = wm_stream(stream);
     Mesh m = make_mesh(nx, ny, nz, dx, dy, dz, xmmin, ymmin, zmmin, zgrid);
     double g = deposit_g(q, wght, nx, ny, nz, dx, dy, dz);
@@ -728,9 +1054,38 @@ int wm_setrho3d(double *rho, int64_t np, const double *xp, const double *yp, con
       WM_HIP(hipMallocAsync((void **)&cnt, sizeof(unsigned long long), s));
       WM_HIP(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), s));
     }
-    hipLaunchKernelGGL(k_setrho, dim3((unsigned)cdiv(np, 256 * DEP_K)), dim3(256), 0, s, rho,
-                       (long long)np, xp, yp, zp, m, g, cnt);
+    BinWork b{};
+    if (w.total) {
+      char *base = (char *)work;
+      b.head = (unsigned int *)base;
+      b.count = (unsigned int *)(base + 256);
+      b.cursor = (unsigned int *)(base + w.cursor);
+      b.list = (unsigned int *)(base + w.list);
+      b.piece = (uint3 *)(base + w.piece);
+      b.x = (double *)(base + w.x);
+      b.y = (double *)(base + w.y);
+      b.z = (double *)(base + w.z);
+      b.ntx = w.ntx;
+      b.nty = w.nty;
+      b.ntiles = w.ntiles;
+    }
+    const int64_t nb = cdiv(np, DEP_PART);
+    hipLaunchKernelGGL(k_setrho, dim3((unsigned)nb), dim3(256), 0, s, rho, (long long)np, xp, yp,
+                       zp, m, g, cnt, b);
     WM_LAUNCHED();
+    if (w.total) {
+      const size_t lds = 2 * sizeof(unsigned int) * (size_t)w.ntiles;
+      if (lds > 60000)  // with its static part beyond the default limit of 64 KB
+        WM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bin_scatter),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      hipLaunchKernelGGL(k_bin_scatter, dim3((unsigned)std::min<int64_t>(nb, 512)),
+                         dim3(BIN_THREADS), lds, s,
+                         (long long)np, xp, yp, zp, m, b);
+      WM_LAUNCHED();
+      hipLaunchKernelGGL(k_bin_deposit, dim3((unsigned)std::min<int64_t>(np, 1024)), dim3(512), 0,
+                         s, rho, m, g, b);
+      WM_LAUNCHED();
+    }
     if (nskipped) {
       unsigned long long h = 0;
       WM_HIP(hipMemcpyAsync(&h, cnt, sizeof(h), hipMemcpyDeviceToHost, s));
@@ -739,6 +1094,14 @@ int wm_setrho3d(double *rho, int64_t np, const double *xp, const double *yp, con
       *nskipped = (int64_t)h;
     }
   });
+}
+
+int wm_setrho3d(double *rho, int64_t np, const double *xp, const double *yp, const double *zp,
+                double zgrid, double q, double wght, int64_t nx, int64_t ny, int64_t nz,
+                double dx, double dy, double dz, double xmmin, double ymmin, double zmmin,
+                int64_t *nskipped, void *stream) {
+  return wm_setrho3d_work(rho, np, xp, yp, zp, zgrid, q, wght, nx, ny, nz, dx, dy, dz, xmmin,
+                          ymmin, zmmin, nskipped, nullptr, 0, stream);
 }
 
 int64_t wm_setrho3d_sorted_worksize(int64_t np, int64_t nx, int64_t ny, int64_t nz) {

@@ -73,7 +73,8 @@ class MultiGrid3D(FieldSolver):
         self._rho = torch.zeros((self.nz + 1, self.ny + 1, self.nx + 1), dtype=torch.float64,
                                 device=self.device)
         self._selfe = None
-        self._work = None
+        self._work = None          # of the sorted deposit
+        self._binwork = None       # of the deposit (counters zero between calls)
         self._nlost = None
         self._cf = None            # conductor field data for f3d.lcorrectede
         self._cf_key = None
@@ -314,9 +315,13 @@ class MultiGrid3D(FieldSolver):
                    z.data_ptr(), zgrid, q, w, self.nx, self.ny, self.nz, self.dx, self.dy,
                    self.dz, self.xmmin, self.ymmin, self.zmmin, self._work.data_ptr(), s)
         else:
-            N.call("wm_setrho3d", self._rho.data_ptr(), n, x.data_ptr(), y.data_ptr(),
+            need = N.lib().wm_setrho3d_worksize(n, self.nx, self.ny, self.nz)
+            if need and (self._binwork is None or self._binwork.numel() < need):
+                self._binwork = torch.zeros(need, dtype=torch.uint8, device=self.device)
+            N.call("wm_setrho3d_work", self._rho.data_ptr(), n, x.data_ptr(), y.data_ptr(),
                    z.data_ptr(), zgrid, q, w, self.nx, self.ny, self.nz, self.dx, self.dy,
-                   self.dz, self.xmmin, self.ymmin, self.zmmin, None, s)
+                   self.dz, self.xmmin, self.ymmin, self.zmmin, None,
+                   self._binwork.data_ptr() if need else None, need, s)
 
     def finalizesourcep(self):
         if self.sourcepfinalized:
