@@ -504,6 +504,14 @@ int wm_unet_conv3(const uint16_t *x, int64_t cin, uint16_t *y, float *yf,
 int wm_unet_conv3_wgrad(const uint16_t *x, int64_t cin, const uint16_t *g,
                         int64_t cout, int64_t D, int64_t H, int64_t W,
                         float *dw, float *db, void *stream);
+/* The same with a workspace of wm_unet_conv3_wgrad_worksize() bytes (0: none
+ * needed), which it overwrites, instead of an allocation per call. */
+int64_t wm_unet_conv3_wgrad_worksize(int64_t cin, int64_t cout, int64_t D,
+                                     int64_t H, int64_t W);
+int wm_unet_conv3_wgrad_work(const uint16_t *x, int64_t cin, const uint16_t *g,
+                             int64_t cout, int64_t D, int64_t H, int64_t W,
+                             float *dw, float *db, void *work,
+                             int64_t worksize, void *stream);
 /* g *= leaky_relu'(y) elementwise (n values). */
 int wm_unet_act_bwd(uint16_t *g, const uint16_t *y, double slope, int64_t n,
                     void *stream);

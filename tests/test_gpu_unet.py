@@ -221,6 +221,44 @@ def test_conv3_weight_gradient_shapes(device, cin, cout, dims):
     assert (db.cpu().to(torch.float64) - b.grad).abs().max() <= 1e-5 * b.grad.abs().max()
 
 
+@pytest.mark.parametrize("cin,cout,dims", [(16, 16, (4, 8, 16)), (48, 16, (5, 9, 11)),
+                                           (16, 64, (2, 3, 240)), (32, 48, (3, 130, 1)),
+                                           (64, 32, (1, 1, 17)), (16, 32, (40, 20, 24))])
+def test_conv3_weight_gradient_forms(device, cin, cout, dims):
+    """The row form of the weight gradient against the tile form, which takes
+    over where an operand is not 16-byte aligned: the same sums in the same
+    order, so dW has the same bits.  Grids of one chunk and of many, rows
+    shorter and longer than a step, and one whose rings need more than 64 KB;
+    an infinite input value reaches the same taps in both."""
+    from warp_amd import _native as N
+    D, H, W = dims
+    g = torch.Generator().manual_seed(cin + cout + W)
+    n = D * H * W
+    x = (torch.randn(n * cin, generator=g)).to(torch.bfloat16)
+    x[cin * (n - 1)] = float("inf")
+    gy = (torch.randn(n * cout, generator=g)).to(torch.bfloat16)
+    s = N.stream_of(device)
+    need = N.lib().wm_unet_conv3_wgrad_worksize(cin, cout, D, H, W)
+    work = torch.empty(need, dtype=torch.uint8, device=device)
+    got = []
+    for off in (0, 4):
+        xd = torch.empty(n * cin + 8, dtype=torch.bfloat16, device=device)[off:off + n * cin]
+        xd.copy_(x)
+        gd = gy.to(device)
+        dw = torch.full((cout * cin * 27,), 0.5, dtype=torch.float32, device=device)
+        db = torch.zeros(cout, dtype=torch.float32, device=device)
+        N.call("wm_unet_conv3_wgrad_work", xd.data_ptr(), cin, gd.data_ptr(), cout, D, H, W,
+               dw.data_ptr(), db.data_ptr(), work.data_ptr(), need, s)
+        got.append((dw.cpu(), db.cpu()))
+    (a, b), (c, d) = got
+    assert torch.equal(torch.isnan(a), torch.isnan(c))
+    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(c)) and not torch.isfinite(a).all()
+    # db: fp32 sums of n bf16 values in two orders
+    assert (b - d).abs().max() <= 1e-5 * n ** 0.5
+    ref = gy.double().reshape(n, cout).sum(0)
+    assert (b.double() - ref).abs().max() <= 1e-5 * n ** 0.5
+
+
 class _RefUNet(torch.nn.Module):
     """The same network in torch (CPU, FP64) with the device weights."""
 

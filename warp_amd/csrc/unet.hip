@@ -596,21 +596,226 @@ __global__ __launch_bounds__(256) void k_wgrad_tiles(const uint16_t *__restrict_
   }
 }
 
-// dw[(co*cin + ci)*27 + tap] += sum over the chunks, in chunk order, of the
-// partial sums of k_wgrad_tiles.
-__global__ __launch_bounds__(256) void k_wgrad_reduce(const float *__restrict__ part, int cin,
-                                                      int cout, long long nchunk,
-                                                      float *__restrict__ dw) {
-  long long o = (long long)blockIdx.x * 256 + threadIdx.x;
-  long long n = 27ll * cout * cin;
-  if (o >= n) return;
-  int tap = (int)(o % 27);
-  long long r = o / 27;
-  int ci = (int)(r % cin), co = (int)(r / cin);
-  int nci = cin >> 4, cit = ci >> 4, cl = ci & 15;
+// 16 voxels of 16 bf16 channels in LDS, transposed: lane l names the 8 bytes
+// l%4 of voxel l/4 and gets channel l%16 of voxels 4(l/16)..+3
+// (ds_read_b64_tr_b16), the K = 16 MFMA operand whose K index is the voxel.
+__device__ inline s4 load_tr(const uint16_t *p) {
+  typedef __attribute__((address_space(3))) s4 lds_s4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p);
+}
+
+// The same sums in the same order (the same bits) where the rows are short
+// enough for LDS: the voxels are taken in memory order, WG_SS at a time.  For
+// each of the three z offsets of the taps the block keeps the part of x
+// within one row and one voxel of the current ones in a ring, as it is in
+// memory ([voxel][16 channels]), so x is read once per z offset instead of
+// once per tap, and written to LDS once, 16 bytes at a time, instead of 27
+// times transposed 2 bytes at a time; the operands are transposed by the LDS
+// read.  Such a read takes an address per voxel: a voxel whose neighbour lies
+// outside the grid reads a zeroed piece of LDS.  One barrier per WG_SS voxels,
+// the next ones' loads in flight meanwhile.  The sums of g (the bias
+// gradient) come from one more MFMA per output block, with ones, in the
+// blocks of the first input block.
+// Bound by the LDS reads and the short chains of each wavefront (64 steps of
+// 16 voxels per block, whose order is kept): 16 -> 16 channels at 128x64x64
+// 129 -> 41 us (0.18 PFLOP/s), 48 -> 16 382 -> 121 us, 32 -> 32 at 64x32x32
+// 42 -> 24 us.  With four wavefronts of seven taps, 55 and 161 us.
+constexpr int WG_SS = 128;
+constexpr int WG_TH = 576;  // nine wavefronts: one for each (dz, dy) of the taps
+
+template <int NT>
+__global__ __launch_bounds__(WG_TH) void k_wgrad_rows(const uint16_t *__restrict__ x, int cin,
+                                                    const uint16_t *__restrict__ g, Dims d,
+                                                    int nvox, int chunk,
+                                                    float *__restrict__ part) {
+  constexpr int COUT = NT * 16;
+  // 16-byte pieces of x and of g per WG_SS voxels, and per thread
+  constexpr int XN = 3 * WG_SS * 2, XPT = (XN + WG_TH - 1) / WG_TH;
+  constexpr int GN = WG_SS * 2 * NT, GPT = (GN + WG_TH - 1) / WG_TH;
+  extern __shared__ __align__(16) uint16_t wlds[];
+  const int L = 2 * d.W + 2 + 2 * WG_SS;     // voxels in a ring
+  uint16_t *zeros = wlds;                    // 16 channels
+  uint16_t *ring = wlds + 16;                // [3][L][16]
+  uint16_t *gbuf = ring + 3 * L * 16;        // [2][NT][WG_SS][16]
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int nci = cin >> 4, cit = blockIdx.x % nci;
+  const int vb = blockIdx.x / nci * chunk, ve = min(vb + chunk, nvox);
+  const int nss = (ve - vb + WG_SS - 1) / WG_SS;
+  const int HW = d.H * d.W;
+  const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+  if (t < 2) *(uint4 *)(zeros + 8 * t) = none;
+  // slot of flat voxel u of ring r: (u - r*HW + HW - (vb - W - 1)) mod L, so
+  // that the first window starts at slot 0
+  auto xpiece = [&](int r, int u, int h) {  // u: voxel relative to the ring's plane offset
+    const long long f = (long long)u + (long long)(r - 1) * HW;
+    return f >= 0 && f < nvox ? *(const uint4 *)(x + f * cin + cit * 16 + 8 * h) : none;
+  };
+  // the first window: [vb - W - 1, vb + WG_SS + W + 1) of each ring
+  const int u0 = vb - d.W - 1, win = WG_SS + 2 * d.W + 2;
+  for (int e = t; e < 3 * win * 2; e += WG_TH) {
+    const int h = e & 1, q = e >> 1, r = q / win, k = q - r * win;
+    *(uint4 *)(ring + (r * L + k) * 16 + 8 * h) = xpiece(r, u0 + k, h);
+  }
+  uint4 xr[XPT], gr[GPT];
+  auto gfetch = [&](int s) {
+#pragma unroll
+    for (int k = 0; k < GPT; k++) {
+      const int e = t + WG_TH * k, v = vb + s * WG_SS + e / (2 * NT);
+      gr[k] = e < GN && v < ve ? *(const uint4 *)(g + (long long)v * COUT + e % (2 * NT) * 8) : none;
+    }
+  };
+  auto gstage = [&](int b) {
+#pragma unroll
+    for (int k = 0; k < GPT; k++) {
+      const int e = t + WG_TH * k, c = e % (2 * NT);
+      if (e < GN)
+        *(uint4 *)(gbuf + ((b * NT + (c >> 1)) * WG_SS + e / (2 * NT)) * 16 + (c & 1) * 8) =
+            gr[k];
+    }
+  };
+  gfetch(0);
+  gstage(0);
+  f4 acc[3][NT], accb[NT];
+#pragma unroll
+  for (int c = 0; c < NT; c++) acc[0][c] = acc[1][c] = acc[2][c] = accb[c] = f4{0.f, 0.f, 0.f, 0.f};
+  const s4 ones = s4{0x3f80, 0x3f80, 0x3f80, 0x3f80};
+  // this wavefront's taps 3 w + dx: ring, offset from the voxel's own slot
+  const int dz = w / 3, dy = w % 3;
+  const uint16_t *myring = ring + dz * L * 16;
+  const int toff = dy * d.W;
+  const int yout = dy == 0 ? 0 : dy == 2 ? d.H - 1 : -1;  // where the neighbour is outside
+  const int zout = dz == 0 ? 0 : dz == 2 ? d.D - 1 : -1;
+  // the voxel this lane reads for others: lane/4 of each 16
+  int v = vb + (lane >> 2);
+  int px = v % d.W, py = v / d.W % d.H, pz = v / HW;
+  int slot = lane >> 2;  // of voxel v - W - 1 (tap offset 0) in its ring
+  const int quarter = (lane & 3) * 4;
+  for (int s = 0; s < nss; s++) {
+    const int b = s & 1;
+    const bool more = s + 1 < nss;
+    if (more) {
+#pragma unroll
+      for (int k = 0; k < XPT; k++) {
+        const int e = t + WG_TH * k, h = e & 1, q = e >> 1, r = q / WG_SS;
+        xr[k] = e < XN ? xpiece(r, u0 + win + s * WG_SS + q % WG_SS, h) : none;
+      }
+      gfetch(s + 1);
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int ks = 0; ks < WG_SS / 16; ks++) {
+      const bool out = py == yout || pz == zout || v >= ve;
+      s4 A[NT];
+#pragma unroll
+      for (int c = 0; c < NT; c++)
+        A[c] = load_tr(gbuf + ((b * NT + c) * WG_SS + ks * 16 + (lane >> 2)) * 16 + quarter);
+      if (w == 4 && cit == 0)
+#pragma unroll
+        for (int c = 0; c < NT; c++)
+          accb[c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[c], ones, accb[c], 0, 0, 0);
+#pragma unroll
+      for (int dx = 0; dx < 3; dx++) {
+        int p = slot + toff + dx;
+        if (p >= L) p -= L;
+        const bool edge = dx == 0 ? px == 0 : dx == 2 ? px == d.W - 1 : false;
+        const s4 B = load_tr((out || edge ? zeros : myring + p * 16) + quarter);
+#pragma unroll
+        for (int c = 0; c < NT; c++)
+          acc[dx][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[c], B, acc[dx][c], 0, 0, 0);
+      }
+      v += 16;
+      px += 16;
+      while (px >= d.W) {
+        px -= d.W;
+        if (++py == d.H) {
+          py = 0;
+          pz++;
+        }
+      }
+      slot += 16;
+      if (slot >= L) slot -= L;
+    }
+    if (more) {
+      // behind the window that the other wavefronts may still be reading
+      const int k0 = (win + s * WG_SS) % L;
+#pragma unroll
+      for (int k = 0; k < XPT; k++) {
+        const int e = t + WG_TH * k, h = e & 1, q = e >> 1, r = q / WG_SS;
+        int p = k0 + q % WG_SS;
+        if (p >= L) p -= L;
+        if (e < XN) *(uint4 *)(ring + (r * L + p) * 16 + 8 * h) = xr[k];
+      }
+      gstage(b ^ 1);
+    }
+  }
+  // lane holds D[4*kg + i][m]: co = c*16 + 4*kg + i, ci = cit*16 + m
+  const int m = lane & 15, kg = lane >> 4;
+  const long long rec = (long long)nci * 27 * COUT * 16 + COUT;
+  float *pr = part + blockIdx.x / nci * rec;
+  float *pb = pr + (long long)cit * 27 * COUT * 16;
+#pragma unroll
+  for (int dx = 0; dx < 3; dx++) {
+    const int tap = 3 * w + dx;
+#pragma unroll
+    for (int c = 0; c < NT; c++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        pb[((long long)tap * COUT + c * 16 + 4 * kg + i) * 16 + m] = acc[dx][c][i];
+  }
+  if (w == 4 && cit == 0 && m == 0)
+#pragma unroll
+    for (int c = 0; c < NT; c++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) pr[rec - COUT + c * 16 + 4 * kg + i] = accb[c][i];
+}
+
+// dw[(co*cin + ci)*27 + tap] and db[co] += the sums over the records of
+// `part` (the blocks' sums, [ci/16][tap][co][16 ci], then with `bias` [co]),
+// in the records' order.  A block takes 64 values: its 16 wavefronts bring
+// RED_REC records at a time to LDS, one adds them up.  One thread per value
+// reading strided through memory, as before, took 166 us for 512 records of
+// 16 -> 16 channels, this 10 us.
+constexpr int RED_REC = 128;
+__global__ __launch_bounds__(1024) void k_wgrad_reduce(const float *__restrict__ part, int cin,
+                                                       int cout, int nrec, int bias,
+                                                       float *__restrict__ dw,
+                                                       float *__restrict__ db) {
+  __shared__ float rows[RED_REC][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int nw = 27 * cout * cin, rec = nw + (bias ? cout : 0);
+  const int e = blockIdx.x * 64 + lane;
   float s = 0.f;
-  for (long long ch = 0; ch < nchunk; ch++)
-    s += part[((ch * nci + cit) * 27 + tap) * (long long)cout * 16 + (long long)co * 16 + cl];
+  for (int r0 = 0; r0 < nrec; r0 += RED_REC) {
+    float v[RED_REC / 16];
+#pragma unroll
+    for (int k = 0; k < RED_REC / 16; k++) {
+      const int r = r0 + w + 16 * k;
+      v[k] = r < nrec && e < rec ? part[(long long)r * rec + e] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RED_REC / 16; k++) rows[w + 16 * k][lane] = v[k];
+    __syncthreads();
+    if (w == 0) {
+      const int n = min(RED_REC, nrec - r0);
+      int r = 0;
+      for (; r + 16 <= n; r += 16) {
+        float q[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) q[k] = rows[r + k][lane];
+#pragma unroll
+        for (int k = 0; k < 16; k++) s += q[k];
+      }
+      for (; r < n; r++) s += rows[r][lane];
+    }
+  }
+  if (w != 0 || e >= rec) return;
+  if (e >= nw) {
+    if (db) db[e - nw] += s;
+    return;
+  }
+  const int cl = e & 15, co = (e >> 4) % cout, q = (e >> 4) / cout;
+  const long long o = ((long long)co * cin + q / 27 * 16 + cl) * 27 + q % 27;
   dw[o] = dw[o] + s;
 }
 
@@ -1116,6 +1321,21 @@ __global__ __launch_bounds__(256) void k_learn_apply(const float *__restrict__ o
 }
 
 inline int nb(long long n) { return (int)std::max<long long>(1, (n + 255) / 256); }
+// The weight gradient's chunks of voxels: about 512 blocks, chunks a multiple
+// of 16 voxels.
+struct WgradSplit {
+  long long nrec, chunk;
+};
+
+inline WgradSplit wgrad_split(int64_t cin, int64_t cout, long long nvox) {
+  const long long nci = cin / 16;
+  WgradSplit p;
+  p.nrec = std::max<long long>(1, std::min<long long>(512 / nci, (nvox + 255) / 256));
+  p.chunk = 16 * ((nvox + 16 * p.nrec - 1) / (16 * p.nrec));
+  p.nrec = (nvox + p.chunk - 1) / p.chunk;
+  return p;
+}
+
 inline bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -1190,8 +1410,16 @@ int wm_unet_conv3(const uint16_t *x, int64_t cin, uint16_t *y, float *yf, int64_
   });
 }
 
-int wm_unet_conv3_wgrad(const uint16_t *x, int64_t cin, const uint16_t *g, int64_t cout,
-                        int64_t D, int64_t H, int64_t W, float *dw, float *db, void *stream) {
+int64_t wm_unet_conv3_wgrad_worksize(int64_t cin, int64_t cout, int64_t D, int64_t H,
+                                     int64_t W) {
+  if (cin < 16 || cout < 16 || cout > 64 || D <= 0 || H <= 0 || W <= 0) return 0;
+  const WgradSplit p = wgrad_split(cin, cout, D * H * W);
+  return (int64_t)sizeof(float) * p.nrec * (27ll * cout * cin + cout);
+}
+
+int wm_unet_conv3_wgrad_work(const uint16_t *x, int64_t cin, const uint16_t *g, int64_t cout,
+                             int64_t D, int64_t H, int64_t W, float *dw, float *db, void *work,
+                             int64_t worksize, void *stream) {
   WM_ENTRY({
     WM_REQUIRE(x && g && dw, "wm_unet_conv3_wgrad: NULL argument");
     WM_REQUIRE(cin % 16 == 0 && cout % 16 == 0 && cin > 0 && cout > 0,
@@ -1199,28 +1427,44 @@ int wm_unet_conv3_wgrad(const uint16_t *x, int64_t cin, const uint16_t *g, int64
     long long nvox = D * H * W;
     Dims d{(int)D, (int)H, (int)W};
     hipStream_t s = wm_stream(stream);
+    if (nvox == 0) return 0;
+    bool bias = false;  // the bias gradient came along
     if (cout <= 64) {
-      // about 512 blocks, chunks a multiple of 16 voxels
-      long long nci = cin / 16;
-      long long nchunk = std::max<long long>(1, std::min<long long>(512 / nci, (nvox + 255) / 256));
-      long long chunk = 16 * ((nvox + 16 * nchunk - 1) / (16 * nchunk));
-      nchunk = (nvox + chunk - 1) / chunk;
-      float *part = nullptr;
-      size_t bytes = sizeof(float) * (size_t)(nchunk * nci * 27 * cout * 16);
-      WM_HIP(hipMallocAsync((void **)&part, bytes, s));
-      unsigned nbk = (unsigned)(nchunk * nci);
-      switch (cout / 16) {
-        case 1: hipLaunchKernelGGL(k_wgrad_tiles<1>, dim3(nbk), dim3(256), 0, s, x, (int)cin, g, d, nvox, chunk, part); break;
-        case 2: hipLaunchKernelGGL(k_wgrad_tiles<2>, dim3(nbk), dim3(256), 0, s, x, (int)cin, g, d, nvox, chunk, part); break;
-        case 3: hipLaunchKernelGGL(k_wgrad_tiles<3>, dim3(nbk), dim3(256), 0, s, x, (int)cin, g, d, nvox, chunk, part); break;
-        default: hipLaunchKernelGGL(k_wgrad_tiles<4>, dim3(nbk), dim3(256), 0, s, x, (int)cin, g, d, nvox, chunk, part); break;
+      const int nt = (int)(cout / 16);
+      const WgradSplit p = wgrad_split(cin, cout, nvox);
+      WM_REQUIRE(work && worksize >= wm_unet_conv3_wgrad_worksize(cin, cout, D, H, W),
+                 "wm_unet_conv3_wgrad: workspace too small");
+      float *part = (float *)work;
+      const dim3 nbk((unsigned)(p.nrec * (cin / 16)));
+      const size_t lds = 2 * (16 + 3 * (2 * (size_t)W + 2 + 2 * WG_SS) * 16 +
+                              2 * (size_t)WG_SS * cout);
+      // The row form where its rings let two blocks share a compute unit, the
+      // 16-byte loads are aligned and 32-bit voxel numbers do
+      bias = lds <= 80 * 1024 && al16(x) && al16(g) && nvox < (1ll << 30);
+      auto run = [&](auto ntc) {
+        constexpr int NT = decltype(ntc)::value;
+        if (bias) {
+          if (lds > 65536)
+            WM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_wgrad_rows<NT>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+          hipLaunchKernelGGL(k_wgrad_rows<NT>, nbk, dim3(WG_TH), lds, s, x, (int)cin, g, d,
+                             (int)nvox, (int)p.chunk, part);
+        } else {
+          hipLaunchKernelGGL(k_wgrad_tiles<NT>, nbk, dim3(256), 0, s, x, (int)cin, g, d, nvox,
+                             p.chunk, part);
+        }
+      };
+      switch (nt) {
+        case 1: run(ic<1>()); break;
+        case 2: run(ic<2>()); break;
+        case 3: run(ic<3>()); break;
+        default: run(ic<4>()); break;
       }
       WM_LAUNCHED();
-      long long n = 27ll * cout * cin;
-      hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, part,
-                         (int)cin, (int)cout, nchunk, dw);
+      const long long rec = 27ll * cout * cin + (bias ? cout : 0);
+      hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((rec + 63) / 64)), dim3(1024), 0, s, part,
+                         (int)cin, (int)cout, (int)p.nrec, (int)bias, dw, db);
       WM_LAUNCHED();
-      WM_HIP(hipFreeAsync(part, s));
     } else {
       int chunk = 4096;
       int nchunk = (int)((nvox + chunk - 1) / chunk);
@@ -1229,11 +1473,24 @@ int wm_unet_conv3_wgrad(const uint16_t *x, int64_t cin, const uint16_t *g, int64
                          (int)cin, g, (int)cout, d, dw, nvox, chunk, nchunk);
       WM_LAUNCHED();
     }
-    if (db) {
+    if (db && !bias) {
       WM_REQUIRE(256 % cout == 0 || cout <= 256, "wm_unet_conv3_wgrad: bad cout");
       hipLaunchKernelGGL(k_bias_grad, dim3(1024), dim3(256), 0, s, g, (int)cout, nvox, db);
       WM_LAUNCHED();
     }
+  });
+}
+
+int wm_unet_conv3_wgrad(const uint16_t *x, int64_t cin, const uint16_t *g, int64_t cout,
+                        int64_t D, int64_t H, int64_t W, float *dw, float *db, void *stream) {
+  WM_ENTRY({
+    hipStream_t s = wm_stream(stream);
+    const int64_t need = wm_unet_conv3_wgrad_worksize(cin, cout, D, H, W);
+    void *part = nullptr;
+    if (need) WM_HIP(hipMallocAsync(&part, (size_t)need, s));
+    const int rc = wm_unet_conv3_wgrad_work(x, cin, g, cout, D, H, W, dw, db, part, need, stream);
+    if (part) WM_HIP(hipFreeAsync(part, s));
+    return rc;
   });
 }
 

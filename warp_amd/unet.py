@@ -153,8 +153,11 @@ class UNet3D:
             nv = d[0] * d[1] * d[2]
             if conv.act:
                 N.call("wm_unet_act_bwd", g.data_ptr(), y.data_ptr(), self.slope, nv * conv.cout, s)
-            N.call("wm_unet_conv3_wgrad", xin.data_ptr(), conv.cin, g.data_ptr(), conv.cout, d[0],
-                   d[1], d[2], conv.gw.data_ptr(), conv.gb.data_ptr(), s)
+            need = N.lib().wm_unet_conv3_wgrad_worksize(conv.cin, conv.cout, *d)
+            work = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+            N.call("wm_unet_conv3_wgrad_work", xin.data_ptr(), conv.cin, g.data_ptr(), conv.cout,
+                   d[0], d[1], d[2], conv.gw.data_ptr(), conv.gb.data_ptr(),
+                   work.data_ptr() if need else None, need, s)
             if not need_dx:
                 return None
             gx = self._t(nv, conv.cin)
