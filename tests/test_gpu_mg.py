@@ -467,6 +467,44 @@ def test_vcycle_tail_same_bits(device, case, monkeypatch):
         np.testing.assert_array_equal(a[2], b[2])
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
+@pytest.mark.parametrize("case", [
+    # mesh, bounds, conductors: tiles cut at the far faces, levels that halve
+    # in some axes only, every boundary type on either side, wrapped windows
+    ((64, 64, 128), (0,) * 6, "pipe_annulus"), ((64, 48, 96), (0, 0, 0, 0, 2, 2), "quads"),
+    ((50, 37, 90), (1, 0, 0, 1, 0, 0), ""), ((41, 66, 54), (1, 1, 1, 1, 1, 0), ""),
+    ((48, 80, 34), (2, 2, 0, 0, 2, 2), ""), ((70, 22, 150), (0, 0, 2, 2, 1, 1), ""),
+    ((33, 100, 47), (0,) * 6, "quads")])
+def test_vcycle_legs_same_bits(device, case, precision, monkeypatch):
+    """Coarse levels as one launch down and one up (tiles with halos in LDS)
+    against the launches step by step: the same phi bit for bit and the same
+    V-cycle counts, cold and warm; and with other smoothing parameters, which
+    go back to the steps."""
+    import warp_amd
+    from warp_amd import configs
+    (nx, ny, nz), bounds, conds = case
+    rng = np.random.default_rng(5)
+    rho = 1e-4 * rng.normal(size=(nz + 1, ny + 1, nx + 1))
+    out = []
+    for nodes in ("0", str(1 << 40)):
+        monkeypatch.setenv("WARPMI_LEG_NODES", nodes)
+        s = _solver(nx, ny, nz, (-0.02, -0.02, 0.0), (0.02, 0.02, 0.08), bounds,
+                    precision=precision, mgmaxiters=12)
+        for g in configs.conductors(conds or None, warp_amd):
+            s.installconductor(g)
+        res = []
+        for f, down in ((1.0, 1), (1.1, 1), (0.9, 2)):
+            s.downpasses = down
+            s.rho = torch.from_numpy(rho * f).to(device)
+            s.solve()
+            res.append((s.mgiters, s.mgerror, s.phi.cpu().numpy().copy()))
+        out.append(res)
+        assert bool(s.leg_levels()) == (nodes != "0")
+    for a, b in zip(*out):
+        assert a[:2] == b[:2]
+        np.testing.assert_array_equal(a[2], b[2])
+
+
 @pytest.mark.parametrize("bounds", [(0,) * 6, (1, 1, 0, 1, 2, 2), (2, 2, 1, 0, 0, 1)])
 def test_residual_wide_rows_match_oracle(device, bounds):
     """residual3d on a level with padded rows (nx = 128: 80 elements per

@@ -11,6 +11,7 @@
 #include "mg3d_kernels.h"
 #include "mg3d_fused.h"
 #include "mg3d_tail.h"
+#include "mg3d_leg.h"
 #include "../../include/warpmi.h"
 
 #include <hip/hip_bf16.h>
@@ -188,6 +189,20 @@ struct CondDev {
   }
 };
 
+// The tiles of one leg (mg3d_leg.h) on a level: the axes (their tables are
+// the level's), the records of the tiles' windows, the launch.
+struct LegTiles {
+  LegAxis a[3];
+  DevBuf<LegTile> tile[3];
+  DevBuf<uint32_t> first;
+  DevBuf<LegRec> rec;
+  int blocks = 0, values = 0;  // values: LDS values of a phi-sized window
+  size_t lds(size_t value) const {
+    return value * (2 * (size_t)values + coarse);
+  }
+  int coarse = 0;  // coarse phi values (up)
+};
+
 struct Level {
   int nx, ny, nz;
   double dx, dy, dz, dxsqi, dysqi, dzsqi;
@@ -234,9 +249,17 @@ struct Level {
   CondDev<double> c64;
   CondDev<float> c32;
   RecKey maskkey;
+  // the transfer tables on the host, and the level's legs
+  std::vector<int> rlo_h[3], rhi_h[3], ej_h[3];
+  bool leg_ok = false;
+  RecKey legkey;
+  DevBuf<uint8_t> legcls;  // class per element (leg_load)
+  LegTiles legdown, legup;
 };
 
 }  // namespace
+
+constexpr long long LEG_NODES = 600000;
 
 struct wm_mg3d {
   int64_t nx, ny, nz;
@@ -312,6 +335,9 @@ struct wm_mg3d {
   DevBuf<TailItem> tailitems;
   DevBuf<TailOp> tailops;
   int dc_double_from = -1;  // levels from here on run in FP64 in the FP32/BF16 V-cycles
+  // levels of at most this many nodes run their legs as one launch each
+  // (WARPMI_LEG_NODES; 0: none), see leg_limit
+  long long leg_nodes = getenv("WARPMI_LEG_NODES") ? atoll(getenv("WARPMI_LEG_NODES")) : LEG_NODES;
   bool tail_used = false;  // the last solve was FP64 and ran the tail
   size_t tail_lds = 0;
   int ncu = 256;                 // compute units of the device
@@ -419,6 +445,8 @@ static void restrict_axis(int n, int nc, int lbm, int lbp, Level &L, int a) {
   L.rstd[a] = std21;
   L.rlo[a].upload(lo);
   L.rhi[a].upload(hi);
+  L.rlo_h[a] = lo;
+  L.rhi_h[a] = hi;
   L.rw[a].upload(w);
   L.rcmin[a] = cmin;
   L.rcmax[a] = cmax;
@@ -442,6 +470,7 @@ static void expand_axis(int n, int nc, int lbm, int lbp, Level &L, int a) {
     w[i] = 1. * (i * nc) / n - j[i];
   }
   L.ej[a].upload(j);
+  L.ej_h[a] = j;
   L.ew[a].upload(w);
   L.elo[a] = lo;
   L.ehi[a] = hi;
@@ -1266,6 +1295,25 @@ static void expand_from(Level &L, T *phi, FI F, const T *pc, CI Cc, const int *s
 }
 
 
+static bool leg_level(const wm_mg3d *h, int level, const Params &P);
+static bool tail_applies(const wm_mg3d *h, int level, const Params &P);
+
+// The error a coarse level's V-cycle ends with: in the second buffer where
+// the level runs by legs.
+template <typename T>
+static T *coarse_phi(wm_mg3d *h, int level, const Params &P) {
+  Level &L = *h->lv[level];
+  return leg_level(h, level, P) ? phib_of<T>(L).p : phi_of<T>(L).p;
+}
+
+// Whether a coarse level's phi has to be zero when its V-cycle starts (the
+// legs and the tail take it as zero without reading it).
+template <typename T>
+static bool needs_zero(const wm_mg3d *h, int level, const Params &P) {
+  if (leg_level(h, level, P)) return false;
+  return !(std::is_same<T, double>::value && tail_applies(h, level, P));
+}
+
 // On a level without voltages (an error level: coarser than the finest, or
 // the finest in the residual-correction form) the pin that starts the
 // first pass after the expansion writes zero at the interior conductor
@@ -1303,11 +1351,11 @@ static void expand_rb(wm_mg3d *h, Level &L, Level &Lc, int level, const Params &
   const uint32_t *imask = fusepin ? L.imask.p : nullptr;
   if ((long long)bpc * cdiv(nzr, 16) >= 1024) {
     hipLaunchKernelGGL((k_expand_rb<S, SC, 16>), dim3(bpc * (int)cdiv(nzr, 16)), dim3(256), 0, s,
-                       phi_of<S>(L).p, L.g, (const SC *)phi_of<SC>(Lc).p, Lc.g, ax, ay, az, jlo,
+                       phi_of<S>(L).p, L.g, (const SC *)coarse_phi<SC>(h, level + 1, P), Lc.g, ax, ay, az, jlo,
                        nj, bpc, imask, skip);
   } else {
     hipLaunchKernelGGL((k_expand_rb<S, SC, 4>), dim3(bpc * (int)cdiv(nzr, 4)), dim3(256), 0, s,
-                       phi_of<S>(L).p, L.g, (const SC *)phi_of<SC>(Lc).p, Lc.g, ax, ay, az, jlo,
+                       phi_of<S>(L).p, L.g, (const SC *)coarse_phi<SC>(h, level + 1, P), Lc.g, ax, ay, az, jlo,
                        nj, bpc, imask, skip);
   }
   WM_LAUNCHED();
@@ -1725,21 +1773,356 @@ static bool coarse_correction(wm_mg3d *h, Level &L, int level, const Params &P,
   // the coarse phi starts at zero: zeroed by the fused kernel's extra
   // blocks, or by k_fill after the separate residual and restriction
   if (fused_restrict_ok(h, L, anyzero)) {
-    resrestrict<S, T, SC>(h, L, Lc, level, P, skip, s, phi_of<SC>(Lc).p, 2 * Lc.g.cs);
+    resrestrict<S, T, SC>(h, L, Lc, level, P, skip, s, phi_of<SC>(Lc).p,
+                          needs_zero<SC>(h, level + 1, P) ? 2 * Lc.g.cs : 0);
   } else {
     residual_rb<S, T>(h, L, level, P, phi_of<S>(L).p, rho_of<S>(L).p, res_of<T>(L).p, 0, skip,
                       s);
     restrict_to<T, SC>(L, (const T *)res_of<T>(L).p, RBIdx{L.g}, rho_of<SC>(Lc).p,
                        RBIdx{Lc.g}, skip, s, Lc.nx, Lc.ny, Lc.nz);
-    hipLaunchKernelGGL((k_fill<SC>), dim3(blocks(2 * Lc.g.cs)), dim3(256), 0, s,
-                       phi_of<SC>(Lc).p, 2 * Lc.g.cs, (SC)0., skip);
-    WM_LAUNCHED();
+    if (needs_zero<SC>(h, level + 1, P)) {
+      hipLaunchKernelGGL((k_fill<SC>), dim3(blocks(2 * Lc.g.cs)), dim3(256), 0, s,
+                         phi_of<SC>(Lc).p, 2 * Lc.g.cs, (SC)0., skip);
+      WM_LAUNCHED();
+    }
   }
   vcycle<SC>(h, level + 1, P, skip, s, true);
   const bool fusepin = P.up > 0 && pin_fusable(h, L, level, P);
   expand_rb<S, SC>(h, L, Lc, level, P, skip, s, fusepin);
   launch_bc<S>(phi_of<S>(L).p, RBIdx{L.g}, L.nx, L.ny, L.nz, h->bounds, 0, 0, skip, s);
   return fusepin;
+}
+
+// ---------------------------------------------------------------------------
+// Legs (mg3d_leg.h).
+
+// Whether the V-cycle on this level, entered with phi at zero, runs as one
+// launch down and one up: a coarse level above the tail, one pass each way.
+static bool leg_level(const wm_mg3d *h, int level, const Params &P) {
+  static const bool tiled_env = getenv("WARPMI_SOR_TILED") != nullptr;
+  if (level < 1 || level + 1 >= (int)h->lv.size() || tiled_env) return false;
+  const Level &L = *h->lv[level];
+  return L.leg_ok && L.legkey.icndbndy == P.icnd && L.legkey.lcndbndy == P.lcnd && P.down == 1 &&
+         P.up == 1 && !fused_ok(h, L, level, P) && !tail_applies(h, level, P);
+}
+
+// The tiles of one leg: windows, launch and the records in each window.
+static bool build_leg(wm_mg3d *h, Level &L, const Level &Lc, LegTiles &D, bool up,
+                      const SubHost *recs) {
+  const int n[3] = {L.nx, L.ny, L.nz}, nc[3] = {Lc.nx, Lc.ny, Lc.nz};
+  const int *b = h->bounds;
+  // fine nodes of a tile, smaller where the level would give few blocks
+  static const int shapes[3][3] = {{16, 8, 8}, {8, 8, 8}, {8, 4, 4}};
+  static const int least[3] = {256, 64, 0};
+  static const int shape_env = getenv("WARPMI_LEG_SHAPE") ? atoi(getenv("WARPMI_LEG_SHAPE")) : -1;
+  struct Win { int w0, w1; };
+  std::vector<Win> win[3];
+  std::vector<LegTile> tiles[3];
+  for (int q = 0; q < 3; q++) {
+    long long blocks = 1;
+    bool fits = true;  // a thread's pairs and LDS
+    D.values = 1;
+    D.coarse = up ? 1 : 0;
+    for (int k = 0; k < 3; k++) {
+      LegAxis &a = D.a[k];
+      a = LegAxis{};
+      a.n = n[k];
+      a.nc = nc[k];
+      a.bm = b[2 * k];
+      a.bp = b[2 * k + 1];
+      a.cmin = L.rcmin[k];
+      a.cmax = L.rcmax[k];
+      a.lo = L.rlo[k].p;
+      a.hi = L.rhi[k].p;
+      a.rw = L.rw[k].p;
+      a.ej = L.ej[k].p;
+      a.ew = L.ew[k].p;
+      const std::vector<int> &lo = L.rlo_h[k], &hi = L.rhi_h[k], &ej = L.ej_h[k];
+      const bool per = a.bm == 2;
+      if (per && (a.n % 2 || a.nc % 2)) return false;
+      if (a.cmax < a.cmin || a.n < 4) return false;
+      a.ts = up ? shapes[q][k] : std::max(1, (shapes[q][k] * a.nc + a.n / 2) / a.n);
+      a.nt = up ? (a.n + a.ts) / a.ts : (a.cmax - a.cmin + a.ts) / a.ts;
+      win[k].clear();
+      tiles[k].clear();
+      auto coarse = [&](int i) {
+        int s = 0;
+        if (per) {
+          if (i < 0) i += a.n, s = -a.nc;
+          if (i >= a.n) i -= a.n, s = a.nc;
+        }
+        return ej[i] + s;
+      };
+      for (int t = 0; t < a.nt; t++) {
+        int w0, w1, o0, o1;  // window; the fine nodes whose phi the tile writes
+        LegTile T{};
+        if (up) {
+          o0 = t * a.ts;
+          o1 = std::min(o0 + a.ts - 1, a.n);
+          w0 = o0 - 2;
+          w1 = o1 + 2;
+        } else {
+          const int c0 = a.cmin + t * a.ts, c1 = std::min(c0 + a.ts - 1, a.cmax);
+          o0 = t == 0 ? 0 : lo[c0];
+          o1 = t == a.nt - 1 ? a.n : lo[c1 + 1] - 1;
+          w0 = lo[c0] - 2;
+          w1 = hi[c1] + 2;
+          // the second half sweep's region has to cover what the tile writes
+          if (o0 < std::max(lo[c0] - 1, 0) || o1 > hi[c1] + 1) return false;
+          for (int c = c0; c <= c1; c++)
+            if (lo[c] < lo[c0] || hi[c] > hi[c1]) return false;
+          T.r0 = lo[c0];
+          T.r1 = hi[c1];
+          T.c0 = c0;
+          T.c1 = c1;
+        }
+        T.own0 = o0;
+        T.own1 = o1;
+        if (per && (w0 < -a.n || w1 > 2 * a.n - 1)) return false;
+        if (!per) {
+          w0 = std::max(w0, 0);
+          w1 = std::min(w1, a.n);
+        }
+        win[k].push_back(Win{w0, w1});
+        a.ext = std::max(a.ext, w1 - w0 + 1);
+        if (up) {
+          const int f = a.bm == 0 && w0 == 0 ? 1 : w0, l = a.bp == 0 && w1 == a.n ? a.n - 1 : w1;
+          if (l < f) return false;
+          T.c0 = coarse(f);
+          T.c1 = coarse(l) + 1;
+          a.cext = std::max(a.cext, T.c1 - T.c0 + 1);
+        }
+        tiles[k].push_back(T);
+      }
+      blocks *= a.nt;
+      D.values *= a.ext;
+      if (up) D.coarse *= a.cext;
+      if (k == 2 && (D.a[0].ext + 1) / 2 * D.a[1].ext * a.ext > LEG_NI * LEG_TH) fits = false;
+      if (a.ext < 4 || a.ext > LEG_WMAX || a.ts > (up ? LEG_WMAX : LEG_CMAX) ||
+          (up && a.cext < 2))
+        return false;
+    }
+    if (blocks >= (1ll << 30)) return false;
+    D.blocks = (int)blocks;
+    fits = fits && D.lds(8) <= 60000;
+    if (fits && (shape_env >= 0 ? q >= shape_env : blocks >= least[q])) break;
+    if (q == 2 && !fits) return false;
+  }
+  for (int k = 0; k < 3; k++) {
+    D.tile[k].upload(tiles[k]);
+    D.a[k].tile = D.tile[k].p;
+  }
+  // tiles and local coordinates of every node, per axis
+  std::vector<std::vector<std::pair<int, int>>> in[3];
+  for (int k = 0; k < 3; k++) {
+    in[k].resize(n[k] + 1);
+    for (int t = 0; t < D.a[k].nt; t++)
+      for (int i = win[k][t].w0; i <= win[k][t].w1; i++) {
+        const int u = b[2 * k] == 2 ? (i % n[k] + n[k]) % n[k] : i;
+        in[k][u].push_back({t, i - win[k][t].w0});
+      }
+  }
+  std::vector<std::vector<LegRec>> lists;
+  long long total = 0;
+  if (recs[0].n() + recs[1].n() > 0) {
+    lists.resize(D.blocks);
+    for (int p = 0; p < 2; p++)
+      for (int i = 0; i < recs[p].n(); i++) {
+        const int *q = &recs[p].pos[3 * i];
+        for (auto &z : in[2][q[2]])
+          for (auto &y : in[1][q[1]])
+            for (auto &x : in[0][q[0]]) {
+              lists[x.first + D.a[0].nt * (y.first + D.a[1].nt * z.first)].push_back(
+                  LegRec{(uint32_t)(x.second | y.second << 8 | z.second << 16),
+                         (uint32_t)p << 31 | (uint32_t)i});
+              total++;
+            }
+      }
+  }
+  std::vector<uint32_t> first(1, 0u);
+  std::vector<LegRec> flat;
+  flat.reserve((size_t)total);
+  for (auto &l : lists) {
+    flat.insert(flat.end(), l.begin(), l.end());
+    first.push_back((uint32_t)flat.size());
+  }
+  D.rec.release();
+  D.first.release();
+  if (total > 0) {
+    D.first.upload(first);
+    D.rec.upload(flat);
+  }
+  return true;
+}
+
+// Legs need: one pin at most per pass that does something a tile can do for
+// itself (no record on an interior point, no Neumann subgrid mirror, no
+// record that zeroes a neighbour's residual), and interior points that the
+// boundary conditions leave interior: beside a Neumann or periodic face the
+// reference copies a neighbour's value over the face before it pins the
+// neighbour, so an interior point next to a face asks for one on it.
+//
+// The largest level that gains: a leg computes its halo again (3-4 points
+// for each of the tile's), against the launches it saves.  Those are three
+// down and three up on a plain level (64x64x128 nodes, FP64: a solve of
+// 128x128x256 1.673 -> 1.595 ms; 80x80x160: 2.798 -> 2.882 with it, 2.818
+// without); one more for the records of conductors (80x80x160: 4.157 -> 3.755
+// ms, 3.775 without it; 128x128x256: slower); boundary launches, pins and the
+// unfused residual with other boundaries (100x100x200, quadrupoles, periodic:
+// 13.07 -> 11.92 ms, 12.11 without it; 128x128x256: 20.22 -> 20.28).
+static long long leg_limit(const wm_mg3d *h, const Level &L) {
+  for (int i = 0; i < 6; i++)
+    if (h->bounds[i] != 0) return 4 * h->leg_nodes;
+  return L.hasmask ? 2 * h->leg_nodes : h->leg_nodes;
+}
+
+static void prepare_legs(wm_mg3d *h, const Params &P) {
+  for (int l = 1; l + 1 < (int)h->lv.size(); l++) {
+    Level &L = *h->lv[l];
+    const long long nodes = (long long)(L.nx + 1) * (L.ny + 1) * (L.nz + 1);
+    RecKey key;
+    key.icndbndy = P.icnd;
+    key.lcndbndy = P.lcnd;
+    if (L.legkey == key) continue;
+    L.legkey = key;
+    L.leg_ok = false;
+    if (!L.coarser || nodes > leg_limit(h, L) || L.sub_on_interior || (P.icnd == 2 && L.neumann))
+      continue;
+    SubHost sor[2];
+    bool ok = true;
+    for (int p = 0; p < 2 && P.lcnd; p++) {
+      sor[p] = build_records(L, l, p, h->bounds, P.mgparam, P.mgform, P.icnd, false, false);
+      const SubHost r = build_records(L, l, p, h->bounds, P.mgparam, P.mgform, P.icnd, true, false);
+      ok = ok && r.pos == sor[p].pos;
+      for (uint32_t z : r.zero) ok = ok && z == 0;
+    }
+    if (ok && L.nint > 0) {
+      std::vector<int> hp(3 * L.nint);
+      WM_HIP(hipMemcpy(hp.data(), L.int_pos.p, sizeof(int) * hp.size(), hipMemcpyDeviceToHost));
+      std::vector<bool> at((size_t)nodes, false);
+      const int n[3] = {L.nx, L.ny, L.nz};
+      auto node = [&](const int *q) {
+        return (size_t)q[0] + (size_t)(L.nx + 1) * (q[1] + (size_t)(L.ny + 1) * q[2]);
+      };
+      for (int i = 0; i < L.nint; i++) at[node(&hp[3 * i])] = true;
+      for (int i = 0; i < L.nint && ok; i++)
+        for (int a = 0; a < 3; a++) {
+          int q[3] = {hp[3 * i], hp[3 * i + 1], hp[3 * i + 2]};
+          auto has = [&](int v) {
+            q[a] = v;
+            return (bool)at[node(q)];
+          };
+          const int v = q[a], bm = h->bounds[2 * a], bp = h->bounds[2 * a + 1];
+          if (bm == 2) {
+            if ((v <= 1 || v >= n[a] - 1) && !(has(0) && has(n[a]))) ok = false;
+          } else {
+            if (bm == 1 && v == 1 && !has(0)) ok = false;
+            if (bp == 1 && v == n[a] - 1 && !has(n[a])) ok = false;
+          }
+        }
+    }
+    L.legcls.release();
+    if (ok && L.hasmask) {
+      std::vector<uint8_t> cls((size_t)(2 * L.g.cs), (uint8_t)LEG_DENSE);
+      if (L.nint > 0) {
+        std::vector<int> hp(3 * L.nint);
+        WM_HIP(hipMemcpy(hp.data(), L.int_pos.p, sizeof(int) * hp.size(), hipMemcpyDeviceToHost));
+        for (int i = 0; i < L.nint; i++)
+          cls[rb_index(L.g, hp[3 * i], hp[3 * i + 1], hp[3 * i + 2])] = LEG_INT;
+      }
+      for (int p = 0; p < 2; p++)
+        for (int i = 0; i < sor[p].n(); i++)
+          cls[rb_index(L.g, sor[p].pos[3 * i], sor[p].pos[3 * i + 1], sor[p].pos[3 * i + 2])] =
+              LEG_REC;
+      L.legcls.upload(cls);
+    }
+    const Level &Lc = *h->lv[l + 1];
+    ok = ok && build_leg(h, L, Lc, L.legdown, false, sor) && build_leg(h, L, Lc, L.legup, true, sor);
+    if (ok != L.leg_ok || ok) {
+      h->drop_graphs();  // captured V-cycles hold the old tables' addresses
+      h->gkey = wm_mg3d::GKey();
+    }
+    L.leg_ok = ok;
+  }
+}
+
+template <typename S>
+static LegArgs<S> leg_args(wm_mg3d *h, Level &L, const Level &Lc, const LegTiles &D,
+                           const Params &P) {
+  LegArgs<S> A{};
+  A.g = L.g;
+  A.gc = Lc.g;
+  for (int k = 0; k < 3; k++) A.a[k] = D.a[k];
+  auto recip = [](int d) { return (uint32_t)(0xffffffffu / (uint32_t)d) + 1u; };
+  for (int i = 0; i < 6; i++)
+    if (h->bounds[i] == 1) A.mirror = 1;
+  A.mhx = recip((D.a[0].ext + 1) / 2);
+  A.my = recip(D.a[1].ext);
+  A.ni = (int)cdiv((D.a[0].ext + 1) / 2 * D.a[1].ext * D.a[2].ext, LEG_TH);
+  A.plain = L.rstd[0] && L.rstd[1] && L.rstd[2];
+  if (D.coarse) {
+    A.mcx = recip(D.a[0].cext);
+    A.mcy = recip(D.a[1].cext);
+  }
+  // the coefficients as halfpass and residual_rb form them
+  const double cst = P.mgparam * 0.5 / (L.dxsqi + L.dysqi + L.dzsqi);
+  A.sx = (S)(L.dxsqi * cst);
+  A.sy = (S)(L.dysqi * cst);
+  A.sz = (S)(L.dzsqi * cst);
+  A.spm1 = (S)(1. - P.mgparam);
+  const double cr = 0.5 / (L.dxsqi + L.dysqi + L.dzsqi);
+  A.rx = (S)(L.dxsqi * P.mgparam * cr);
+  A.ry = (S)(L.dysqi * P.mgparam * cr);
+  A.rz = (S)(L.dzsqi * P.mgparam * cr);
+  A.mgparam = (S)P.mgparam;
+  A.ff = L.ff;
+  A.cls = L.legcls.p;
+  if (P.lcnd && D.rec.p) {
+    A.first = D.first.p;
+    A.rec = D.rec.p;
+    CondDev<S> &C = cond_of<S>(L);
+    for (int c = 0; c < 2; c++) {
+      A.sor[c] = C.sor[c].view();
+      A.res[c] = C.res[0][c].view();
+    }
+  }
+  return A;
+}
+
+template <typename S, typename SC>
+static void leg_pair(wm_mg3d *h, Level &L, int level, const Params &P, const int *skip,
+                     hipStream_t s) {
+  Level &Lc = *h->lv[level + 1];
+  if (L.hasmask) ensure_records<S>(h, L, level, P, true, 0);
+  hipLaunchKernelGGL((k_leg_down<S, SC>), dim3(L.legdown.blocks), dim3(LEG_TH),
+                     L.legdown.lds(sizeof(S)), s, leg_args<S>(h, L, Lc, L.legdown, P),
+                     (const S *)rho_of<S>(L).p, phi_of<S>(L).p, rho_of<SC>(Lc).p, skip);
+  WM_LAUNCHED();
+  if (needs_zero<SC>(h, level + 1, P)) {
+    hipLaunchKernelGGL((k_fill<SC>), dim3(blocks(2 * Lc.g.cs)), dim3(256), 0, s,
+                       phi_of<SC>(Lc).p, 2 * Lc.g.cs, (SC)0., skip);
+    WM_LAUNCHED();
+  }
+  vcycle<SC>(h, level + 1, P, skip, s, true);
+  hipLaunchKernelGGL((k_leg_up<S, SC>), dim3(L.legup.blocks), dim3(LEG_TH),
+                     L.legup.lds(sizeof(S)), s, leg_args<S>(h, L, Lc, L.legup, P),
+                     (const S *)rho_of<S>(L).p, (const S *)phi_of<S>(L).p,
+                     (const SC *)coarse_phi<SC>(h, level + 1, P), phib_of<S>(L).p, skip);
+  WM_LAUNCHED();
+}
+
+template <typename S>
+static void leg_down_up(wm_mg3d *h, Level &L, int level, const Params &P, const int *skip,
+                        hipStream_t s) {
+  if constexpr (std::is_same<S, double>::value) {
+    leg_pair<double, double>(h, L, level, P, skip, s);
+  } else {
+    // the coarsest level and those the tail can hold are solved in FP64
+    if (level + 2 == (int)h->lv.size() || level + 1 == h->dc_double_from)
+      leg_pair<S, double>(h, L, level, P, skip, s);
+    else
+      leg_pair<S, S>(h, L, level, P, skip, s);
+  }
 }
 
 template <typename S>
@@ -1770,6 +2153,12 @@ static void vcycle(wm_mg3d *h, int level, const Params &P, const int *skip, hipS
                          s, (const TailLevel *)h->tailtab.p, (const TailItem *)h->tailitems.p,
                          (const TailOp *)h->tailops.p, h->tail.run, skip);
       WM_LAUNCHED();
+      return;
+    }
+  }
+  if constexpr (!std::is_same<S, bf16>::value) {
+    if (zeroed && leg_level(h, level, P)) {
+      leg_down_up<S>(h, L, level, P, skip, s);
       return;
     }
   }
@@ -2089,6 +2478,7 @@ int wm_mg3d_set_conductors(wm_mg3d *h, const wm_conductor_lists *c) {
       L.imask.release();
       L.c64.reset();
       L.c32.reset();
+      L.legkey = RecKey();
     }
     h->conductors_set = false;
     h->last_ok = false;
@@ -2181,6 +2571,7 @@ int wm_mg3d_solve(wm_mg3d *h, double *phi, double *rho, double mgparam, int64_t 
     }
     h->save64.alloc_rb(2 * L0.g.cs);
     prepare_tail(h, P);
+    prepare_legs(h, P);
     h->tail_used = h->tail.on && prec == WM_PREC_FP64 && mgmaxiters > 0;
     // Inputs.
     WM_HIP(hipEventRecord(h->ev_in, us));
@@ -2430,6 +2821,15 @@ int wm_mg3d_tail_start(const wm_mg3d *h, int64_t *level) {
   WM_ENTRY({
     WM_REQUIRE(h && level, "wm_mg3d_tail_start: NULL argument");
     *level = h->tail_used ? h->tail.start : -1;
+  });
+}
+
+int wm_mg3d_leg_levels(const wm_mg3d *h, int64_t *levels) {
+  WM_ENTRY({
+    WM_REQUIRE(h && levels, "wm_mg3d_leg_levels: NULL argument");
+    *levels = 0;
+    for (size_t l = 1; l < h->lv.size() && l < 63; l++)
+      if (h->lv[l]->leg_ok) *levels |= 1ll << l;
   });
 }
 

@@ -414,6 +414,13 @@ class MultiGrid3D(FieldSolver):
         N.call("wm_mg3d_tail_start", self._h, C.byref(r))
         return int(r.value)
 
+    def leg_levels(self):
+        """The coarse levels whose V-cycle runs as one launch down and one
+        up, as far as the last solve's parameters allow."""
+        r = C.c_int64(0)
+        N.call("wm_mg3d_leg_levels", self._h, C.byref(r))
+        return [l for l in range(63) if r.value >> l & 1]
+
     def _phi_version(self):
         """(version, address) of phi, or None where torch keeps no version
         counter (tensors made under torch.inference_mode)."""
