@@ -231,6 +231,7 @@ struct Level {
   DevBuf<double> ew[3];
   int elo[3], ehi[3];
   bool rstd[3] = {false, false, false};  // restriction windows are the plain 2:1 ones
+  bool rhalf[3] = {false, false, false};  // and so at any faces
   // conductors
   int nint = 0;
   DevBuf<int> int_pos;
@@ -241,6 +242,11 @@ struct Level {
   // an active subgrid record sits on an interior (pinned) point, so the
   // pin after each half sweep is not a no-op
   bool sub_on_interior = false;
+  // faces_of (-1: not looked at yet), the interior points and, per element, the
+  // sides across which it reads one before the pin
+  int faces = -1;
+  std::vector<int> int_h;
+  std::vector<uint8_t> raw_h;
   std::vector<int> subpos_h[2];
   std::vector<double> subdels_h[2], subvolt_h[2];
   DevBuf<int> subpos_d[2];
@@ -318,7 +324,7 @@ struct wm_mg3d {
   int sor_form = getenv("WARPMI_SOR_FUSED") ? std::min(2, std::max(0, atoi(getenv("WARPMI_SOR_FUSED")))) : 0;
   bool conductors_set = false;
   // The coarse end of the FP64 V-cycle in one launch (k_vtail): levels
-  // start..nlevels-1, described by the device table tailtab (fixed address,
+  // start..nlevels-1, described by the device table taildesc (fixed address,
   // contents rewritten between solves when they change).  The levels whose
   // arrays fit in tail_lds bytes of LDS qualify (WARPMI_TAIL_LDS sets a
   // smaller budget; 0 switches the tail off).
@@ -326,14 +332,13 @@ struct wm_mg3d {
     bool on = false;
     int start = -1;
     TailRun run{};
-    std::vector<TailLevel> host;  // contents of tailtab
-    std::vector<TailItem> items;  // contents of tailitems
-    std::vector<TailOp> ops;      // contents of tailops
+    std::vector<unsigned char> desc;  // contents of taildesc
+    std::vector<TailItem> items;      // contents of tailitems
     int down = -1, up = -1;       // the pass counts the steps are for
   } tail;
-  DevBuf<TailLevel> tailtab;
+  DevBuf<unsigned char> taildesc;
   DevBuf<TailItem> tailitems;
-  DevBuf<TailOp> tailops;
+  DevBuf<uint32_t> tailimage;  // of the launch's LDS
   int dc_double_from = -1;  // levels from here on run in FP64 in the FP32/BF16 V-cycles
   // levels of at most this many nodes run their legs as one launch each
   // (WARPMI_LEG_NODES; 0: none), see leg_limit
@@ -443,6 +448,11 @@ static void restrict_axis(int n, int nc, int lbm, int lbp, Level &L, int a) {
     std21 = lo[ic] == 2 * ic - 1 && hi[ic] == 2 * ic + 1 && w[5 * ic] == 0.5 &&
             w[5 * ic + 1] == 1. && w[5 * ic + 2] == 0.5;
   L.rstd[a] = std21;
+  bool half = n == 2 * nc;
+  for (int ic = cmin; ic <= cmax && half; ic++)
+    half = lo[ic] == 2 * ic - 1 && hi[ic] == 2 * ic + 1 && w[5 * ic] == 0.5 &&
+           w[5 * ic + 1] == 1. && w[5 * ic + 2] == 0.5;
+  L.rhalf[a] = half;
   L.rlo[a].upload(lo);
   L.rhi[a].upload(hi);
   L.rlo_h[a] = lo;
@@ -1535,6 +1545,67 @@ static bool pp_applies(const wm_mg3d *h, const Params &P) {
   return !off && !tiled_env && P.down >= 1 && P.up >= 1 && !fused_ok(h, *h->lv[0], 0, P);
 }
 
+// What the interior points of a level ask of a form without boundary launches,
+// in which the neighbours across a Neumann or periodic face are found by
+// address and plane 0 of a periodic axis stands for plane n.  After a half
+// sweep and its boundary conditions the guard points hold what the address
+// finds, and the pins after the half sweeps change nothing, unless a point of
+// plane 0 is interior and its image is not.  Between the expansion and the
+// first half sweep after it the reference fills the guard points before it
+// pins: there an interior point next to a face counts across it with its value
+// from before the pin (unless the face's point is interior itself).
+enum {
+  FACES_BEYOND = 1,  // some point counts across a face with its value before the pin
+  FACES_UNEVEN = 2,  // an interior point of plane n whose image on plane 0 is not
+  FACES_NO = 4,      // the form does not give the reference's values
+};
+static int faces_of(const wm_mg3d *h, Level &L) {
+  if (L.faces >= 0) return L.faces;
+  const int n[3] = {L.nx, L.ny, L.nz};
+  int f = 0;
+  bool face = false;
+  for (int a = 0; a < 3; a++) {
+    face = face || h->bounds[2 * a] != 0 || h->bounds[2 * a + 1] != 0;
+    if (h->bounds[2 * a] == 2 && n[a] % 2) f |= FACES_NO;  // the colours do not meet
+  }
+  if (!f && face && L.nint > 0) {
+    // (downloads the points: once per conductor set)
+    L.int_h.resize(3 * L.nint);
+    WM_HIP(hipMemcpy(L.int_h.data(), L.int_pos.p, sizeof(int) * L.int_h.size(),
+                     hipMemcpyDeviceToHost));
+    L.raw_h.assign((size_t)(2 * L.g.cs), 0);
+    std::vector<bool> at((size_t)(L.nx + 1) * (L.ny + 1) * (L.nz + 1), false);
+    auto node = [&](const int *q) {
+      return (size_t)q[0] + (size_t)(L.nx + 1) * (q[1] + (size_t)(L.ny + 1) * q[2]);
+    };
+    for (int i = 0; i < L.nint; i++) at[node(&L.int_h[3 * i])] = true;
+    for (int i = 0; i < L.nint; i++)
+      for (int a = 0; a < 3; a++) {
+        int q[3] = {L.int_h[3 * i], L.int_h[3 * i + 1], L.int_h[3 * i + 2]};
+        // the face's point at coordinate v reads this one across side s
+        auto reads = [&](int v, int s) {
+          q[a] = v;
+          if (at[node(q)]) return;
+          f |= FACES_BEYOND;
+          L.raw_h[rb_index(L.g, q[0], q[1], q[2])] |= (uint8_t)(1 << (2 * a + s));
+        };
+        auto has = [&](int v) {
+          q[a] = v;
+          return (bool)at[node(q)];
+        };
+        const int v = q[a], bm = h->bounds[2 * a], bp = h->bounds[2 * a + 1];
+        if (bm == 1 && v == 1) reads(0, 0);
+        if (bp == 1 && v == n[a] - 1) reads(n[a], 1);
+        if (bm != 2) continue;
+        if (v == n[a] - 1) reads(0, 0);
+        if (v == 0 && !has(n[a])) f |= FACES_NO;
+        if (v == n[a] && !has(0)) f |= FACES_UNEVEN;
+      }
+  }
+  L.faces = f;
+  return f;
+}
+
 // The FP64 V-cycle's tail (k_vtail) for the parameters P: the first level
 // from 1 on with at most tail_nodes nodes, and every level from there on
 // using the half sweeps (the fused pass swaps buffers, which the table does
@@ -1571,14 +1642,19 @@ static void prepare_tail(wm_mg3d *h, const Params &P) {
   for (int start = 1; start < nlev; start++) {
     std::vector<TailLevel> tab;
     std::vector<TailItem> items;
-    int off = 0, gw = 0;
-    // an LDS region of `words` (even offset); gathered from src when given
+    std::vector<TailPass> passes;
+    int off = 0;
+    // an LDS region of `words` (even offset); copied from src when given
     auto region = [&](const void *src, long long words) -> int {
       const int o = off;
       off += (int)((words + 1) & ~1ll);
       if (src && words > 0) {
-        items.push_back(TailItem{(const uint32_t *)src, o, (int)words, gw, 0});
-        gw += (int)((words + TAIL_GB - 1) / TAIL_GB * TAIL_GB);
+        TailItem it;
+        std::memset(&it, 0, sizeof(it));
+        it.src = (const uint32_t *)src;
+        it.dst = o;
+        it.words = (int)words;
+        items.push_back(it);
       }
       return o;
     };
@@ -1601,62 +1677,119 @@ static void prepare_tail(wm_mg3d *h, const Params &P) {
       std::memset(&t, 0, sizeof(t));
       t.g = L.g;
       t.phi = L.phi64.p;
-      const long long n2 = 2 * L.g.cs;
-      // level arrays: only the first level's rho comes from HBM (its phi is
-      // zero, the others' phi and rho are written by the restriction, and
-      // the points of res that no residual writes are zero)
-      t.lphi = region(nullptr, 2 * n2);
-      t.lrho = region(l == start ? (const void *)L.rho64.p : nullptr, 2 * n2);
-      if (L.coarser) t.lres = region(nullptr, 2 * n2);
+      CondDev<double> &C = cond_of<double>(L);
+      const bool mirror = P.icnd == 2 && L.neumann;
+      const bool res1 = !(L.sub_on_interior && L.nint > 0) && !C.res[0][0].anyzero &&
+                        !C.res[0][1].anyzero;
+      const int faces = faces_of(h, L);
+      const bool wrap = !mirror && !L.sub_on_interior && res1 && !(faces & FACES_NO) &&
+                        (L.nint == 0 || L.imask.p) &&
+                        !((faces & FACES_UNEVEN) && L.hasmask && !P.lcnd);
       LoopRange sr = sor_range(L, b), rr = res_range(L, b);
+      if (wrap) {  // the planes n of periodic axes are written with the planes 0
+        if (b[0] == 2) sr.ixmax = rr.ixmax = L.nx - 1;
+        if (b[2] == 2) sr.iymax = rr.iymax = L.ny - 1;
+        if (b[4] == 2) sr.izmax = rr.izmax = L.nz - 1;
+      }
       const int srv[6] = {sr.ixmin, sr.ixmax, sr.iymin, sr.iymax, sr.izmin, sr.izmax};
       const int rrv[6] = {rr.ixmin, rr.ixmax, rr.iymin, rr.iymax, rr.izmin, rr.izmax};
-      for (int i = 0; i < 6; i++) {
-        t.sr[i] = srv[i];
-        t.rr[i] = rrv[i];
-      }
-      // padded element and row counts of the ranges (powers of two)
-      auto lg2 = [](int n) {
-        int k = 0;
-        while ((1 << k) < n) k++;
-        return k;
-      };
-      t.ssh[0] = lg2((sr.ixmax + 1) / 2 - (sr.ixmin + 1) / 2 + 1);
-      t.ssh[1] = lg2(sr.iymax - sr.iymin + 1);
-      t.rsh[0] = lg2((rr.ixmax + 1) / 2 - (rr.ixmin + 1) / 2 + 1);
-      t.rsh[1] = lg2(rr.iymax - rr.iymin + 1);
-      // the coefficients as halfpass and residual_rb form them
+      // the coefficients as residual_rb forms them
       const double cst = P.mgparam * 0.5 / (L.dxsqi + L.dysqi + L.dzsqi);
-      t.sc[0] = L.dxsqi * cst;
-      t.sc[1] = L.dysqi * cst;
-      t.sc[2] = L.dzsqi * cst;
-      t.sc[3] = 1. - P.mgparam;
       const double cr = 0.5 / (L.dxsqi + L.dysqi + L.dzsqi);
-      t.rc[0] = L.dxsqi * P.mgparam * cr;
-      t.rc[1] = L.dysqi * P.mgparam * cr;
-      t.rc[2] = L.dzsqi * P.mgparam * cr;
       t.rs[0] = P.mgparam * L.dxsqi * cr;
       t.rs[1] = P.mgparam * L.dysqi * cr;
       t.rs[2] = P.mgparam * L.dzsqi * cr;
-      CondDev<double> &C = cond_of<double>(L);
       int f = 0;
-      const bool mirror = P.icnd == 2 && L.neumann;
-      if (L.sub_on_interior || periodic || mirror) f |= TAIL_PIN_AFTER;
+      if (wrap) f |= TAIL_WRAP | (periodic ? TAIL_PER : 0);
+      if (!wrap && (L.sub_on_interior || periodic || mirror)) f |= TAIL_PIN_AFTER;
       if (mirror) f |= TAIL_MIRROR;
-      if (L.sub_on_interior && L.nint > 0) f |= TAIL_SPLIT;
-      if (L.coarser && P.up > 0 && pin_fusable(h, L, l, P)) f |= TAIL_FUSEPIN;
-      if (L.hasmask) f |= TAIL_HASMASK;
-      if (!(L.sub_on_interior && L.nint > 0) && !C.res[0][0].anyzero && !C.res[0][1].anyzero)
-        f |= TAIL_RES1;
+      // (with TAIL_WRAP nothing comes between the expansion and the pin)
+      if (L.coarser && P.up > 0 && L.nint > 0 && L.imask.p &&
+          (wrap || pin_fusable(h, L, l, P)))
+        f |= TAIL_FUSEPIN;
+      if (wrap && (f & TAIL_FUSEPIN) && (faces & FACES_BEYOND)) f |= TAIL_GUARD;
+      if (L.coarser && L.rhalf[0] && L.rhalf[1] && L.rhalf[2]) f |= TAIL_HALF;
+      if (res1) f |= TAIL_RES1;
       t.flags = f;
-      if (L.hasmask) t.lmask = region(L.mask.p, (long long)L.mask.n);
       if (f & TAIL_FUSEPIN) t.limask = region(L.imask.p, (long long)L.imask.n);
       t.nint = L.nint;
       if (L.nint > 0) t.lint = region(L.int_pos.p, 3ll * L.nint);
-      for (int c = 0; c < 2; c++) {
-        t.sor[c] = sub(P.lcnd ? C.sor[c].view() : none, false);
-        t.rsub[c] = sub(L.hasmask && L.coarser ? C.res[0][c].view() : none, true);
+      // the two half sweeps, the two colours of the residual
+      const RBGeom &g = L.g;
+      for (int k = 0; k < (L.coarser ? 4 : 2); k++) {
+        const int c = k & 1;
+        const bool res = k >= 2;
+        const int *r = res ? rrv : srv;
+        TailPass p;
+        std::memset(&p, 0, sizeof(p));
+        p.W = g.W;
+        p.pl = g.W * g.PY;
+        p.res = res;
+        TailItem it;
+        std::memset(&it, 0, sizeof(it));
+        it.kind = TIM_POINTS;
+        it.colour = c;
+        it.g = g;
+        for (int a = 0; a < 6; a++) it.r[a] = r[a], it.b[a] = wrap ? b[a] : 0;
+        // (the ranges agree, and with them the points: one table)
+        const bool same = res && std::memcmp(srv, rrv, sizeof(srv)) == 0;
+        const long long nj = (r[1] + 1) / 2 - (r[0] + 1) / 2 + 1;
+        p.n = r[1] >= r[0] && r[3] >= r[2] && r[5] >= r[4]
+                  ? (int)(nj * (r[3] - r[2] + 1) * (r[5] - r[4] + 1))
+                  : 0;
+        if (same) {
+          p.tab = passes[passes.size() - 2].tab;
+        } else if (p.n > 0) {
+          it.src = L.hasmask ? L.mask.p : nullptr;
+          it.dst = p.tab = region(nullptr, p.n);
+          it.words = p.n;
+          items.push_back(it);
+        }
+        const int st[3] = {1, g.W, g.W * g.PY};
+        for (int a = 0; a < 3; a++) {
+          const int n = a == 0 ? g.nx : a == 1 ? g.ny : g.nz;
+          // (x: in elements of the other colour's row)
+          if (a == 0) {
+            p.f[0] = b[0] == 2 ? n >> 1 : 1;
+            p.f[1] = (n >> 1) - ((n + 1) >> 1);
+          } else {
+            p.f[2 * a] = b[2 * a] == 2 ? st[a] * (n - 1) : st[a];
+            p.f[2 * a + 1] = -st[a];
+          }
+          p.im[a] = a == 0 ? n >> 1 : st[a] * n;
+        }
+        const SubList<double> v = !res ? (P.lcnd ? C.sor[c].view() : none)
+                                       : (L.hasmask && res1 ? C.res[0][c].view() : none);
+        if (v.n > 0) {
+          p.nr = v.n;
+          it.kind = TIM_RECORDS;
+          it.src = (const uint32_t *)v.pos;
+          it.dst = p.rtab = region(nullptr, v.n);
+          it.words = v.n;
+          items.push_back(it);
+          p.modes = region(v.modes, v.n);
+          p.k = region(v.k, 12ll * v.n);
+          p.denom = region(v.denom, 2ll * v.n);
+          if (res) p.fac = region(v.fac, 2ll * v.n);
+        }
+        if (!res) {
+          p.c[0] = p.r[0] = L.dxsqi * cst;
+          p.c[1] = p.r[1] = L.dysqi * cst;
+          p.c[2] = p.r[2] = L.dzsqi * cst;
+          p.c[3] = p.r[3] = 1. - P.mgparam;
+        } else {
+          p.c[0] = L.dxsqi * P.mgparam * cr;
+          p.c[1] = L.dysqi * P.mgparam * cr;
+          p.c[2] = L.dzsqi * P.mgparam * cr;
+          p.c[3] = -P.mgparam;
+          for (int a = 0; a < 3; a++) p.r[a] = t.rs[a];
+          p.r[3] = P.mgparam;
+        }
+        passes.push_back(p);
       }
+      if (!res1)
+        for (int c = 0; c < 2; c++)
+          t.rsub[c] = sub(L.hasmask && L.coarser ? C.res[0][c].view() : none, true);
       for (int p = 0; p < 2; p++) {
         t.nsub[p] = (int)(L.subpos_h[p].size() / 3);
         t.subpos[p] = L.subpos_d[p].p;
@@ -1669,77 +1802,129 @@ static void prepare_tail(wm_mg3d *h, const Params &P) {
                               region(L.rw[a].p, 2ll * (long long)L.rw[a].n), L.rcmin[a],
                               L.rcmax[a]};
           t.ea[a] = TailAxisE{region(L.ej[a].p, (long long)L.ej[a].n),
-                              region(L.ew[a].p, 2ll * (long long)L.ew[a].n), L.elo[a], L.ehi[a]};
+                              region(L.ew[a].p, 2ll * (long long)L.ew[a].n), L.elo[a],
+                              wrap && b[2 * a] == 2 ? rrv[2 * a + 1] : L.ehi[a]};
         }
         t.ff = L.ff;
+        auto recip = [](int d) { return d > 1 ? (uint32_t)((1ull << 32) / (unsigned)d + 1) : 0u; };
+        t.mr[0] = recip(L.rcmax[0] - L.rcmin[0] + 1);
+        t.mr[1] = recip(L.rcmax[1] - L.rcmin[1] + 1);
+        t.me[0] = recip(t.ea[0].hi - t.ea[0].lo + 1);
+        t.me[1] = recip(t.ea[1].hi - t.ea[1].lo + 1);
       }
       tab.push_back(t);
     }
-    if ((size_t)off * 4 > h->tail_lds || (int)items.size() > TAIL_MAX_ITEMS) continue;
+    // the level arrays (phi starts at zero, rho is copied or written by the
+    // restriction, the points of res that no residual writes are zero)
+    const int tab_words = off = (off + 3) & ~3;
+    bool fits = true;
+    for (int l = start, k = 0; l < nlev; l++) {
+      const Level &L = *h->lv[l];
+      TailLevel &t = tab[l - start];
+      const long long n2 = 4 * L.g.cs;
+      fits = fits && L.g.cs < TW_EVEN && (long long)off + 3 * n2 < (1ll << 28);
+      if (!fits) break;
+      t.lphi = region(nullptr, n2);
+      t.lrho = region(nullptr, n2);
+      if (L.coarser) t.lres = region(nullptr, n2);
+      const int cw = (int)(2 * L.g.cs);
+      for (int q = 0; q < (L.coarser ? 4 : 2); q++, k++) {
+        TailPass &p = passes[k];
+        const int c = q & 1;
+        p.own = t.lphi + c * cw;
+        p.oth = t.lphi + (1 - c) * cw;
+        p.rho = t.lrho + c * cw;
+        p.dst = q >= 2 ? t.lres + c * cw : p.own;
+      }
+    }
+    off = (off + 3) & ~3;
+    if (!fits || (size_t)off * 4 > h->tail_lds || (int)items.size() > TAIL_MAX_ITEMS) continue;
     // the steps, in the order vcycle and its callees launch them for these
     // levels (phi of the first level starts at zero)
     std::vector<TailOp> ops;
     const int nl = (int)tab.size();
     const bool anybc = b[0] || b[1] || b[2] || b[3] || b[4] || b[5];
-    auto pass = [&](int l, bool pin) {
+    // (levels before the coarsest have four passes each)
+    auto pass = [&](int l, bool pin, bool guards) {
       const TailLevel &t = tab[l];
-      const bool sweeps = t.sr[3] >= t.sr[2] && t.sr[5] >= t.sr[4];
-      if (pin) ops.push_back(TailOp{TOP_PIN, l, 0, 0});
+      const LoopRange r = sor_range(*h->lv[start + l], b);
+      // nothing (records included) where the y or z range is empty
+      const bool sweeps = r.iymax >= r.iymin && r.izmax >= r.izmin;
+      // a pin where there is something to pin
+      const bool pins = t.nint > 0 || (t.flags & TAIL_MIRROR);
+      if (pin && pins) ops.push_back(TailOp{TOP_PIN, l, 0, 0});
       for (int c = 0; c < 2; c++) {
-        ops.push_back(TailOp{TOP_HALF, l, c, 0});
-        if (sweeps && (t.flags & TAIL_PIN_AFTER)) ops.push_back(TailOp{TOP_PIN, l, 0, 0});
-        if (anybc) ops.push_back(TailOp{TOP_BCPHI, l, 0, 0});
+        const int by_address = (t.flags & TAIL_WRAP) && !(guards && c == 0) ? TPASS_FACES : 0;
+        if (sweeps) ops.push_back(TailOp{TOP_PASS, l, by_address | TPASS_SYNC, 4 * l + c});
+        if (pins && sweeps && (t.flags & TAIL_PIN_AFTER)) ops.push_back(TailOp{TOP_PIN, l, 0, 0});
+        if (anybc && !(t.flags & TAIL_WRAP)) ops.push_back(TailOp{TOP_BCPHI, l, 0, 0});
       }
     };
     for (int l = 0; l < nl; l++) {
-      for (int i = 0; i < P.down; i++) pass(l, i > 0);
+      const int f = tab[l].flags;
+      for (int i = 0; i < P.down; i++) pass(l, i > 0, false);
       if (l + 1 < nl) {
-        ops.push_back(TailOp{TOP_RESID, l, 0, 0});
+        for (int c = 0; c < 2; c++)
+          ops.push_back(TailOp{TOP_PASS, l, (f & TAIL_WRAP ? TPASS_FACES : 0) | (c ? TPASS_SYNC : 0),
+                               4 * l + 2 + c});
+        if (!(f & TAIL_RES1)) ops.push_back(TailOp{TOP_RESREC, l, 0, 0});
+        if (anybc && !(f & TAIL_WRAP)) ops.push_back(TailOp{TOP_BCRES, l, 0, 0});
         ops.push_back(TailOp{TOP_RESTRICT, l, 0, 0});
       }
     }
     for (int l = nl - 1; l >= 0; l--) {
-      bool fusepin = false;
+      bool fusepin = false, guards = false;
       if (l + 1 < nl) {
         ops.push_back(TailOp{TOP_EXPAND, l, 0, 0});
         fusepin = tab[l].flags & TAIL_FUSEPIN;
+        guards = tab[l].flags & TAIL_GUARD;
       }
-      for (int i = 0; i < P.up; i++) pass(l, !(fusepin && i == 0));
+      for (int i = 0; i < P.up; i++) pass(l, !(fusepin && i == 0), guards && i == 0);
     }
     if ((int)ops.size() > TAIL_MAX_OPS) return;
     TailRun run{};
     run.nops = (int)ops.size();
+    run.tab_words = tab_words;
     for (int i = 0; i < 6; i++) run.b[i] = b[i];
     run.mgparam = P.mgparam;
     run.lds_words = off;
-    run.nitems = (int)items.size();
-    run.gather_words = gw;
-    if (h->tailtab.n < (size_t)nlev) h->tailtab.alloc((size_t)nlev);
+    run.rho0 = (const uint32_t *)h->lv[start]->rho64.p;
+    run.lrho0 = tab[0].lrho;
+    run.rho_words = (int)(4 * h->lv[start]->g.cs);
+    const size_t words = (h->tail_lds + 15) / 16 * 4;
+    if (h->tailimage.n < words) h->tailimage.alloc(words);
+    run.image = h->tailimage.p;
+    // steps, passes and levels as one buffer
+    auto up64 = [](size_t n) { return (n + 63) / 64 * 64; };
+    std::vector<unsigned char> desc(up64(sizeof(TailOp) * ops.size()) +
+                                    up64(sizeof(TailPass) * passes.size()) +
+                                    up64(sizeof(TailLevel) * tab.size()));
+    run.at_pass = (int)up64(sizeof(TailOp) * ops.size());
+    run.at_level = run.at_pass + (int)up64(sizeof(TailPass) * passes.size());
+    run.desc_bytes = (int)desc.size();
+    if (!ops.empty()) std::memcpy(desc.data(), ops.data(), sizeof(TailOp) * ops.size());
+    std::memcpy(desc.data() + run.at_pass, passes.data(), sizeof(TailPass) * passes.size());
+    std::memcpy(desc.data() + run.at_level, tab.data(), sizeof(TailLevel) * tab.size());
+    const size_t most = up64(sizeof(TailOp) * TAIL_MAX_OPS) +
+                        (size_t)nlev * up64(4 * sizeof(TailPass) + sizeof(TailLevel)) + 128;
+    if (h->taildesc.n < most) h->taildesc.alloc(most);
     if (h->tailitems.n < (size_t)TAIL_MAX_ITEMS) h->tailitems.alloc((size_t)TAIL_MAX_ITEMS);
-    if (h->tailops.n < (size_t)TAIL_MAX_OPS) h->tailops.alloc((size_t)TAIL_MAX_OPS);
     const bool same =
-        h->tail.host.size() == tab.size() && h->tail.items.size() == items.size() &&
-        h->tail.ops.size() == ops.size() &&
-        std::memcmp(h->tail.host.data(), tab.data(), sizeof(TailLevel) * tab.size()) == 0 &&
+        h->tail.desc == desc && h->tail.items.size() == items.size() &&
         (items.empty() ||
-         std::memcmp(h->tail.items.data(), items.data(), sizeof(TailItem) * items.size()) == 0) &&
-        (ops.empty() || std::memcmp(h->tail.ops.data(), ops.data(), sizeof(TailOp) * ops.size()) == 0);
+         std::memcmp(h->tail.items.data(), items.data(), sizeof(TailItem) * items.size()) == 0);
     if (!same) {
-      // captured V-cycles hold the old step count and gather sizes by value
+      // captured V-cycles hold the old step count and sizes by value
       h->drop_graphs();
       h->gkey = wm_mg3d::GKey();
       WM_HIP(hipStreamSynchronize(h->s));
-      WM_HIP(hipMemcpy(h->tailtab.p, tab.data(), sizeof(TailLevel) * tab.size(),
-                       hipMemcpyHostToDevice));
+      WM_HIP(hipMemset(h->tailimage.p, 0, sizeof(uint32_t) * h->tailimage.n));
+      WM_HIP(hipMemcpy(h->taildesc.p, desc.data(), desc.size(), hipMemcpyHostToDevice));
       if (!items.empty())
         WM_HIP(hipMemcpy(h->tailitems.p, items.data(), sizeof(TailItem) * items.size(),
                          hipMemcpyHostToDevice));
-      if (!ops.empty())
-        WM_HIP(hipMemcpy(h->tailops.p, ops.data(), sizeof(TailOp) * ops.size(),
-                         hipMemcpyHostToDevice));
-      h->tail.host = tab;
+      h->tail.desc = desc;
       h->tail.items = items;
-      h->tail.ops = ops;
     }
     h->tail.down = P.down;
     h->tail.up = P.up;
@@ -1929,11 +2114,12 @@ static bool build_leg(wm_mg3d *h, Level &L, const Level &Lc, LegTiles &D, bool u
     for (int p = 0; p < 2; p++)
       for (int i = 0; i < recs[p].n(); i++) {
         const int *q = &recs[p].pos[3 * i];
+        const uint32_t raw = L.raw_h.empty() ? 0u : L.raw_h[rb_index(L.g, q[0], q[1], q[2])];
         for (auto &z : in[2][q[2]])
           for (auto &y : in[1][q[1]])
             for (auto &x : in[0][q[0]]) {
               lists[x.first + D.a[0].nt * (y.first + D.a[1].nt * z.first)].push_back(
-                  LegRec{(uint32_t)(x.second | y.second << 8 | z.second << 16),
+                  LegRec{(uint32_t)(x.second | y.second << 8 | z.second << 16) | raw << 24,
                          (uint32_t)p << 31 | (uint32_t)i});
               total++;
             }
@@ -1957,10 +2143,8 @@ static bool build_leg(wm_mg3d *h, Level &L, const Level &Lc, LegTiles &D, bool u
 
 // Legs need: one pin at most per pass that does something a tile can do for
 // itself (no record on an interior point, no Neumann subgrid mirror, no
-// record that zeroes a neighbour's residual), and interior points that the
-// boundary conditions leave interior: beside a Neumann or periodic face the
-// reference copies a neighbour's value over the face before it pins the
-// neighbour, so an interior point next to a face asks for one on it.
+// record that zeroes a neighbour's residual), and neighbours across faces that
+// the interior points leave to addresses (faces_of).
 //
 // The largest level that gains: a leg computes its halo again (3-4 points
 // for each of the tile's), against the launches it saves.  Those are three
@@ -1996,31 +2180,7 @@ static void prepare_legs(wm_mg3d *h, const Params &P) {
       ok = ok && r.pos == sor[p].pos;
       for (uint32_t z : r.zero) ok = ok && z == 0;
     }
-    if (ok && L.nint > 0) {
-      std::vector<int> hp(3 * L.nint);
-      WM_HIP(hipMemcpy(hp.data(), L.int_pos.p, sizeof(int) * hp.size(), hipMemcpyDeviceToHost));
-      std::vector<bool> at((size_t)nodes, false);
-      const int n[3] = {L.nx, L.ny, L.nz};
-      auto node = [&](const int *q) {
-        return (size_t)q[0] + (size_t)(L.nx + 1) * (q[1] + (size_t)(L.ny + 1) * q[2]);
-      };
-      for (int i = 0; i < L.nint; i++) at[node(&hp[3 * i])] = true;
-      for (int i = 0; i < L.nint && ok; i++)
-        for (int a = 0; a < 3; a++) {
-          int q[3] = {hp[3 * i], hp[3 * i + 1], hp[3 * i + 2]};
-          auto has = [&](int v) {
-            q[a] = v;
-            return (bool)at[node(q)];
-          };
-          const int v = q[a], bm = h->bounds[2 * a], bp = h->bounds[2 * a + 1];
-          if (bm == 2) {
-            if ((v <= 1 || v >= n[a] - 1) && !(has(0) && has(n[a]))) ok = false;
-          } else {
-            if (bm == 1 && v == 1 && !has(0)) ok = false;
-            if (bp == 1 && v == n[a] - 1 && !has(n[a])) ok = false;
-          }
-        }
-    }
+    ok = ok && !(faces_of(h, L) & (FACES_NO | FACES_UNEVEN));
     L.legcls.release();
     if (ok && L.hasmask) {
       std::vector<uint8_t> cls((size_t)(2 * L.g.cs), (uint8_t)LEG_DENSE);
@@ -2034,6 +2194,9 @@ static void prepare_legs(wm_mg3d *h, const Params &P) {
         for (int i = 0; i < sor[p].n(); i++)
           cls[rb_index(L.g, sor[p].pos[3 * i], sor[p].pos[3 * i + 1], sor[p].pos[3 * i + 2])] =
               LEG_REC;
+      // the sides across which a point reads an interior one before its pin
+      for (size_t e = 0; e < L.raw_h.size(); e++)
+        if (cls[e] != LEG_INT) cls[e] |= (uint8_t)(L.raw_h[e] << 2);
       L.legcls.upload(cls);
     }
     const Level &Lc = *h->lv[l + 1];
@@ -2150,8 +2313,7 @@ static void vcycle(wm_mg3d *h, int level, const Params &P, const int *skip, hipS
     // levels from the tail's start on, entered with phi at zero
     if (zeroed && level > 0 && tail_applies(h, level, P)) {
       hipLaunchKernelGGL(k_vtail, dim3(1), dim3(1024), sizeof(uint32_t) * h->tail.run.lds_words,
-                         s, (const TailLevel *)h->tailtab.p, (const TailItem *)h->tailitems.p,
-                         (const TailOp *)h->tailops.p, h->tail.run, skip);
+                         s, (const unsigned char *)h->taildesc.p, h->tail.run, skip);
       WM_LAUNCHED();
       return;
     }
@@ -2401,12 +2563,12 @@ int wm_mg3d_create(wm_mg3d **out, int64_t nx, int64_t ny, int64_t nz, double dx,
     WM_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev));
     if (ncu > 0) h->ncu = ncu;
     if (lds > 0) h->lds_per_cu = (size_t)lds;
-    // LDS of the V-cycle tail: what one workgroup may hold, less the item
-    // list and 1 KB
+    // LDS of the V-cycle tail: what one workgroup may hold, less 7 KB (the
+    // line decides which levels the FP32 and BF16 V-cycles hold in FP64)
     {
       int blk = 0;
       WM_HIP(hipDeviceGetAttribute(&blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-      const size_t fixed = sizeof(TailItem) * TAIL_MAX_ITEMS + 1024;
+      const size_t fixed = 7168;
       size_t cap = (size_t)blk > fixed ? (size_t)blk - fixed : 0;
       if (getenv("WARPMI_TAIL_LDS")) cap = std::min<size_t>(cap, (size_t)atoll(getenv("WARPMI_TAIL_LDS")));
       if (cap > 65536 && hipFuncSetAttribute(reinterpret_cast<const void *>(&k_vtail),
@@ -2479,6 +2641,8 @@ int wm_mg3d_set_conductors(wm_mg3d *h, const wm_conductor_lists *c) {
       L.c64.reset();
       L.c32.reset();
       L.legkey = RecKey();
+      L.faces = -1;
+      L.raw_h.clear();
     }
     h->conductors_set = false;
     h->last_ok = false;
@@ -2620,6 +2784,11 @@ int wm_mg3d_solve(wm_mg3d *h, double *phi, double *rho, double mgparam, int64_t 
     }
     hipLaunchKernelGGL(k_state_reset, dim3(1), dim3(1), 0, s, h->state.p);
     WM_LAUNCHED();
+    if (h->tail.on && !h->tail.items.empty()) {
+      hipLaunchKernelGGL(k_tail_image, dim3((unsigned)h->tail.items.size()), dim3(256), 0, s,
+                         (const TailItem *)h->tailitems.p, h->tailimage.p);
+      WM_LAUNCHED();
+    }
     if (prec == WM_PREC_FP64)
       zero_interior_res<double>(h, dc ? P2of(P) : P, s);
     else

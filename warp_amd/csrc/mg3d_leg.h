@@ -59,8 +59,8 @@ struct LegAxis {
   const LegTile *tile;
 };
 
-// A conductor record of a tile's window: local coordinates (8 bits each) and
-// (colour << 31) | index.
+// A conductor record of a tile's window: local coordinates (8 bits each) with
+// the sides of LEGP_RAW (6 bits), and (colour << 31) | index.
 struct LegRec {
   uint32_t at, rec;
 };
@@ -76,7 +76,7 @@ struct LegArgs {
   T sx, sy, sz, spm1;              // half sweep
   T rx, ry, rz, mgparam;           // residual
   double ff;
-  const uint8_t *cls;              // class per element (NULL: all dense)
+  const uint8_t *cls;              // class per element and the sides of LEGP_RAW << 2 (NULL: all dense)
   const uint32_t *first;           // a tile's records: rec[first[t]] .. rec[first[t+1]]
   const LegRec *rec;               // NULL: none
   SubList<T> sor[2], res[2];
@@ -116,10 +116,22 @@ struct LegNb {
 
 // A point's word: the steps it takes part in (0-3: the steps' regions lie one
 // inside the other), the faces it mirrors at, whether the tile writes it,
-// interior conductor point, record.
-enum { LEGP_DEPTH = 3, LEGP_MIRROR = 4, LEGP_OWN = 256, LEGP_INT = 512, LEGP_REC = 1024 };
+// interior conductor point, record, the sides across which it reads an
+// interior point before its pin.
+enum {
+  LEGP_DEPTH = 3,
+  LEGP_MIRROR = 4,
+  LEGP_OWN = 256,
+  LEGP_INT = 512,
+  LEGP_REC = 1024,
+  LEGP_RAW = 2048
+};
 
-__device__ inline LegNb leg_nb(uint32_t p, int ex, int sz) {
+// raw (not 0): the first half sweep after the expansion.  The reference fills
+// the guard points before it pins, so a point on a face reads an interior
+// neighbour across it as it was before the pin; that value stands raw elements
+// behind the point, in the place of its rho.
+__device__ inline LegNb leg_nb(uint32_t p, int ex, int sz, int raw) {
   LegNb q{-1, 1, -ex, ex, -sz, sz};
   if (p & (63u * LEGP_MIRROR)) {
     if (p & (LEGP_MIRROR << 0)) q.xm = 1;
@@ -128,6 +140,14 @@ __device__ inline LegNb leg_nb(uint32_t p, int ex, int sz) {
     if (p & (LEGP_MIRROR << 3)) q.yp = -ex;
     if (p & (LEGP_MIRROR << 4)) q.zm = sz;
     if (p & (LEGP_MIRROR << 5)) q.zp = -sz;
+  }
+  if (raw && (p & (63u * LEGP_RAW))) {
+    if (p & (LEGP_RAW << 0)) q.xm += raw;
+    if (p & (LEGP_RAW << 1)) q.xp += raw;
+    if (p & (LEGP_RAW << 2)) q.ym += raw;
+    if (p & (LEGP_RAW << 3)) q.yp += raw;
+    if (p & (LEGP_RAW << 4)) q.zm += raw;
+    if (p & (LEGP_RAW << 5)) q.zp += raw;
   }
   return q;
 }
@@ -224,8 +244,10 @@ __device__ inline void leg_load(const LegArgs<T> &A, const LegWin *r0, const Leg
       const bool sw = q & LEGP_DEPTH;
       // the conductor points take no part; interior ones where their phi or
       // residual is asked for
-      if (sw && cl[i][p] != LEG_DENSE)
-        q = (q & LEGP_OWN) | (cl[i][p] == LEG_REC           ? LEGP_REC
+      const int cls = cl[i][p] & 3;
+      if (UP && sw && cls == LEG_DENSE) q |= (uint32_t)(cl[i][p] >> 2) * LEGP_RAW;
+      if (sw && cls != LEG_DENSE)
+        q = (q & LEGP_OWN) | (cls == LEG_REC                ? LEGP_REC
                               : UP || (q & LEGP_DEPTH) == 3u ? LEGP_INT
                                                              : 0u);
       // (the second point of a row's last pair may be the next row's first)
@@ -279,10 +301,11 @@ __device__ inline void leg_load_record(const LegArgs<T> &A, LegRec q, LegRecord<
 
 // The records of colour c inside r: half sweep (sor_record) or, with res, the
 // residual (residual_record).  first: phi is zero everywhere, the
-// neighbours, which may lie outside the window, are read from the point.
+// neighbours, which may lie outside the window, are read from the point.  raw:
+// leg_nb.
 template <typename T, bool RES>
 __device__ inline void leg_records(const LegArgs<T> &A, const LegWin *w, const LegWin *r, int c,
-                                   bool res, bool first, T *ph, T *rh, int rec0, int nrec,
+                                   bool res, bool first, int raw, T *ph, T *rh, int rec0, int nrec,
                                    const LegRecord<T, RES> &mine) {
   const int ex = A.a[0].ext, ey = A.a[1].ext, sz = ex * ey;
   // (the last threads first: they own the fewest pairs)
@@ -290,12 +313,12 @@ __device__ inline void leg_records(const LegArgs<T> &A, const LegWin *w, const L
   for (int i = LEG_TH - 1 - (int)threadIdx.x; i < nrec; i += LEG_TH) {
     LegRecord<T, RES> R = mine;
     if (i >= LEG_TH) leg_load_record<T, RES>(A, A.rec[rec0 + i], R);
-    const int lx = R.at & 255u, ly = (R.at >> 8) & 255u, lz = R.at >> 16;
+    const int lx = R.at & 255u, ly = (R.at >> 8) & 255u, lz = (R.at >> 16) & 255u;
     const int x = w[0].w0 + lx, y = w[1].w0 + ly, z = w[2].w0 + lz;
     if ((int)(R.rec >> 31) != c || !leg_in(r, x, y, z)) continue;
     const int e = lx + ex * (ly + ey * lz);
     LegNb q{0, 0, 0, 0, 0, 0};
-    if (!first) q = leg_nb(leg_mirror(A, x, y, z), ex, sz);
+    if (!first) q = leg_nb(leg_mirror(A, x, y, z) | (R.at >> 24) * LEGP_RAW, ex, sz, raw);
     uint32_t m = R.modes;
     T k[6];
 #pragma unroll
@@ -320,17 +343,18 @@ __device__ inline void leg_records(const LegArgs<T> &A, const LegWin *w, const L
   }
 }
 
-// A half sweep of colour c for the dense points of at least the given depth.
+// A half sweep of colour c for the dense points of at least the given depth
+// (raw: leg_nb).
 template <typename T>
 __device__ inline void leg_sweep(const LegArgs<T> &A, const LegPts &P, int c, uint32_t depth,
-                                 T *ph, const T *rh) {
+                                 int raw, T *ph, const T *rh) {
   const int ex = A.a[0].ext, sz = ex * A.a[1].ext;
 #pragma unroll
   for (int i = 0; i < LEG_NI; i++) {
     const uint32_t p = P.w[i][c];
     if ((p & LEGP_DEPTH) < depth) continue;
     const int e = leg_el(P, i, c);
-    const LegNb q = leg_nb(p, ex, sz);
+    const LegNb q = leg_nb(p, ex, sz, raw);
     ph[e] = rh[e] + (ph[e + q.xm] + ph[e + q.xp]) * A.sx + (ph[e + q.ym] + ph[e + q.yp]) * A.sy +
             (ph[e + q.zm] + ph[e + q.zp]) * A.sz + A.spm1 * ph[e];
   }
@@ -430,11 +454,11 @@ __global__ __launch_bounds__(LEG_TH) void k_leg_down(LegArgs<S> A, const S *__re
   if (nrec) {
     // (records read only their own rho and phi here: written above by other
     // threads, hence the barrier)
-    leg_records<T, true>(A, w, w, 0, false, true, ph, rh, rec0, nrec, mine);
+    leg_records<T, true>(A, w, w, 0, false, true, 0, ph, rh, rec0, nrec, mine);
     __syncthreads();
   }
-  leg_sweep<T>(A, P, 1, 2u, ph, rh);
-  if (nrec) leg_records<T, true>(A, w, b, 1, false, false, ph, rh, rec0, nrec, mine);
+  leg_sweep<T>(A, P, 1, 2u, 0, ph, rh);
+  if (nrec) leg_records<T, true>(A, w, b, 1, false, false, 0, ph, rh, rec0, nrec, mine);
   __syncthreads();
   leg_store<T>(A, w, P, ph, phi);
   // the residual, in the place of rho (each point reads its own rho alone)
@@ -446,14 +470,14 @@ __global__ __launch_bounds__(LEG_TH) void k_leg_down(LegArgs<S> A, const S *__re
       if (p & LEGP_INT) rh[leg_el(P, i, c)] = (T)0.;
       if ((p & LEGP_DEPTH) < 3u) continue;
       const int e = leg_el(P, i, c);
-      const LegNb q = leg_nb(p, ex, sz);
+      const LegNb q = leg_nb(p, ex, sz, 0);
       rh[e] = rh[e] + (ph[e + q.xm] + ph[e + q.xp]) * A.rx + (ph[e + q.ym] + ph[e + q.yp]) * A.ry +
               (ph[e + q.zm] + ph[e + q.zp]) * A.rz - ph[e] * A.mgparam;
     }
   if (nrec)
 #pragma unroll 1
     for (int c = 0; c < 2; c++)
-      leg_records<T, true>(A, w, r, c, true, false, ph, rh, rec0, nrec, mine);
+      leg_records<T, true>(A, w, r, c, true, false, 0, ph, rh, rec0, nrec, mine);
   __syncthreads();
   // restriction (restrict_point, k_restrict_t)
   const int nx = tl[0].c1 - tl[0].c0 + 1, ny = tl[1].c1 - tl[1].c0 + 1,
@@ -598,14 +622,15 @@ __global__ __launch_bounds__(LEG_TH) void k_leg_up(LegArgs<S> A, const S *__rest
                   wx * (one - wy) * wz * o[fz + 1] + (one - wx) * wy * wz * o[fz + fx] +
                   wx * wy * wz * o[fz + fx + 1];
       ph[e] = p & LEGP_INT ? (T)0. : v;
+      if (p & LEGP_INT) rh[e] = v;  // (before the pin: leg_nb's raw)
     }
   }
   __syncthreads();
-  leg_sweep<T>(A, P, 0, 2u, ph, rh);
-  if (nrec) leg_records<T, false>(A, w, c, 0, false, false, ph, rh, rec0, nrec, mine);
+  leg_sweep<T>(A, P, 0, 2u, nw, ph, rh);
+  if (nrec) leg_records<T, false>(A, w, c, 0, false, false, nw, ph, rh, rec0, nrec, mine);
   __syncthreads();
-  leg_sweep<T>(A, P, 1, 3u, ph, rh);
-  if (nrec) leg_records<T, false>(A, w, own, 1, false, false, ph, rh, rec0, nrec, mine);
+  leg_sweep<T>(A, P, 1, 3u, 0, ph, rh);
+  if (nrec) leg_records<T, false>(A, w, own, 1, false, false, 0, ph, rh, rec0, nrec, mine);
   __syncthreads();
   leg_store<T>(A, w, P, ph, out);
 }
