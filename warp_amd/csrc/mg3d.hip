@@ -323,6 +323,7 @@ struct wm_mg3d {
   // (wm_mg3d_set_sor_form; WARPMI_SOR_FUSED=1 or 2 sets the default)
   int sor_form = getenv("WARPMI_SOR_FUSED") ? std::min(2, std::max(0, atoi(getenv("WARPMI_SOR_FUSED")))) : 0;
   bool conductors_set = false;
+  bool res0_steady = false;  // this solve's res64 of the finest level holds its fixed zeros
   // The coarse end of the FP64 V-cycle in one launch (k_vtail): levels
   // start..nlevels-1, described by the device table taildesc (fixed address,
   // contents rewritten between solves when they change).  The levels whose
@@ -760,7 +761,26 @@ static void launch_bc(T *u, Idx I, int nx, int ny, int nz, const int *b, int lwd
   int need[3];
   for (int a = 0; a < 3; a++)
     need[a] = (b[2 * a] != 0 || b[2 * a + 1] != 0 || lwd || lzd);
-  int dims[3] = {nx, ny, nz};
+  const int dims[3] = {nx, ny, nz};
+  // two or three axes at once, unless Dirichlet guards are asked for, an axis
+  // is so short that its points lie on their own images, or (a caller's
+  // bounds) it is periodic on one side only
+  bool shell = !lwd && !lzd && need[0] + need[1] + need[2] > 1;
+  long long points = 0;
+  BcFaces B;
+  for (int a = 0; a < 3; a++) {
+    shell = shell && dims[a] >= 2 && (b[2 * a] == 2) == (b[2 * a + 1] == 2);
+    const int m = b[2 * a] == 2 ? 3 : (b[2 * a] == 1) + (b[2 * a + 1] == 1);
+    points += m * (long long)(dims[a == 0 ? 1 : 0] + 3) * (dims[a == 2 ? 1 : 2] + 3);
+    B.b[2 * a] = b[2 * a];
+    B.b[2 * a + 1] = b[2 * a + 1];
+  }
+  if (shell && points < (1ll << 30)) {
+    hipLaunchKernelGGL((k_bc_shell<T, Idx>), dim3(blocks(points)), dim3(256), 0, s, u, I, nx, ny,
+                       nz, B, skip);
+    WM_LAUNCHED();
+    return;
+  }
   for (int a = 0; a < 3; a++) {
     if (!need[a]) continue;
     int na = a == 0 ? ny : nx, nb = a == 2 ? ny : nz;
@@ -768,7 +788,6 @@ static void launch_bc(T *u, Idx I, int nx, int ny, int nz, const int *b, int lwd
     hipLaunchKernelGGL((k_bc_axis<T, Idx>), dim3(blocks(n)), dim3(256), 0, s, u, I, a, nx, ny,
                        nz, b[2 * a], b[2 * a + 1], lwd, lzd, skip);
     WM_LAUNCHED();
-    (void)dims;
   }
 }
 
@@ -893,12 +912,12 @@ static void halfpass(wm_mg3d *h, Level &L, int level, const Params &P, int c,
   }
   // cond_potmg after the sweep (f3d_mgrid.F:2276-2285).  The dense sweep
   // skips every interior point and the pass starts with a pin, so the
-  // pin is a no-op unless a subgrid record or a periodic wrap can write an
-  // interior point, or Neumann subgrid ghosts must be mirrored.  A half
-  // sweep called alone (inpass false) always pins.
-  const int *b = h->bounds;
-  bool periodic = b[0] == 2 || b[2] == 2 || b[4] == 2;
-  if (!inpass || L.sub_on_interior || periodic || (P.icnd == 2 && L.neumann)) {
+  // pin is a no-op unless a subgrid record can write an interior point, or
+  // Neumann subgrid ghosts must be mirrored.  (On plane n of a periodic axis,
+  // which the conditions before wrote, the pin changes interior points, but
+  // the conditions that follow it write the whole plane again.)  A half sweep
+  // called alone (inpass false) always pins.
+  if (!inpass || L.sub_on_interior || (P.icnd == 2 && L.neumann)) {
     int usevolt = (level == 0 && P.mgform == 1);
     pin_and_mirror<S>(h, L, level, P, phi, usevolt, skip, s);
   }
@@ -1962,7 +1981,7 @@ static bool coarse_correction(wm_mg3d *h, Level &L, int level, const Params &P,
                           needs_zero<SC>(h, level + 1, P) ? 2 * Lc.g.cs : 0);
   } else {
     residual_rb<S, T>(h, L, level, P, phi_of<S>(L).p, rho_of<S>(L).p, res_of<T>(L).p, 0, skip,
-                      s);
+                      s, std::is_same<S, double>::value && level == 0 && h->res0_steady);
     restrict_to<T, SC>(L, (const T *)res_of<T>(L).p, RBIdx{L.g}, rho_of<SC>(Lc).p,
                        RBIdx{Lc.g}, skip, s, Lc.nx, Lc.ny, Lc.nz);
     if (needs_zero<SC>(h, level + 1, P)) {
@@ -2793,8 +2812,16 @@ int wm_mg3d_solve(wm_mg3d *h, double *phi, double *rho, double mgparam, int64_t 
       zero_interior_res<double>(h, dc ? P2of(P) : P, s);
     else
       zero_interior_res<float>(h, Params{P.mgparam, 2, P.down, P.up, P.lcnd, P.icnd}, s);
-    // the fixed zeros of the defect-correction source (its residual runs
-    // in the steady form)
+    // the fixed zeros of the finest level's residual (which then runs in the
+    // steady form) ...
+    h->res0_steady = prec == WM_PREC_FP64 && L0.coarser && L0.res64.p;
+    if (h->res0_steady) {
+      CondDev<double> &C = cond_of<double>(L0);
+      const bool anyzero = L0.hasmask && (C.res[0][0].anyzero || C.res[0][1].anyzero);
+      h->res0_steady = !fused_restrict_ok(h, L0, anyzero);
+    }
+    if (h->res0_steady) residual_zeros<double>(h, L0, L0.res64.p, s);
+    // ... and of the defect-correction source
     if (dc) {
       if (prec == WM_PREC_FP64) residual_zeros<double>(h, L0, L0.rho64.p, s);
       else if (prec == WM_PREC_FP32_DC) residual_zeros<float>(h, L0, L0.rho32.p, s);
