@@ -66,8 +66,8 @@ __device__ inline uint32_t pk_bf16(float a, float b) {
 
 // Forward convolution.  A block (4 wavefronts) owns a tile of 16 x VT x 4
 // output voxels (x, y, z): wavefront w takes z plane z0 + w and its VT
-// rows of 16 voxels, for all NT*16 output channels (VT*NT accumulators of
-// 16 voxels x 16 channels).  Per 16-channel input block the block copies
+// rows of 16 voxels, for NT*16 of the output channels (VT*NT accumulators of
+// 16 voxels x 16 channels; blockIdx.y counts the groups of channels).  Per 16-channel input block the block copies
 // the tile and its one-voxel halo, 18 x (VT+2) x 6 voxels of 16 channels,
 // into LDS (zeros outside the grid), then runs 15 MFMA steps; in step s a
 // lane reads its A operand (voxel m of its row, shifted by the tap of step
@@ -75,13 +75,27 @@ __device__ inline uint32_t pk_bf16(float a, float b) {
 // packed weights, each B operand feeding the VT row tiles.  out = act(conv +
 // bias), act the leaky ReLU of slope `slope` (1 = identity); bias may be
 // NULL.
+//
+// On the coarse levels a block is a chain of latencies (the tile, then the
+// weights of each step) and there are few blocks.  With VT = 1 a block takes
+// 16 output channels, which makes as many more blocks as there are groups,
+// and asks for the weights of all 15 steps at once; the tile of the next
+// input block is read during the steps (AHEAD).  32x16x16 voxels, 48 -> 48
+// channels 21.6 -> 12.3 us, 16x8x8, 64 -> 64 29 -> 8.2 us.  With more rows the
+// reading ahead has to be worth its registers, 24 a thread at VT = 4 and 14 at
+// 2: it is with three channel groups (64x32x32, 48 -> 48 45 -> 34 us in the
+// network) and with two rows (112 -> 80 channels 79 -> 74 us), not with one
+// or two groups (80 -> 32 channels at 64x32x32 32 -> 48 us) or four (64 -> 64
+// at 96x64x64 133 -> 153 us): these stage in turn.
 template <int NT, int VT>
 __global__ __launch_bounds__(256) void k_conv3(const uint16_t *__restrict__ x, int cin,
                                                uint16_t *__restrict__ y, float *__restrict__ yf,
                                                Dims d, const uint16_t *__restrict__ wq,
                                                const float *__restrict__ bias, float slope,
-                                               int ntx, int nty) {
+                                               int ntx, int nty, int ncout) {
   constexpr int HX = 18, HY = VT + 2, HZ = 6, HV = HX * HY * HZ;
+  constexpr bool AHEAD = VT <= 2 || NT == 3;
+  constexpr int UN = VT == 1 ? 15 : 3;
   __shared__ __align__(16) uint16_t tile[HV * 16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int m = lane & 15, kg = lane >> 4;
@@ -90,29 +104,52 @@ __global__ __launch_bounds__(256) void k_conv3(const uint16_t *__restrict__ x, i
   b /= ntx;
   const int ty = b % nty, tz = b / nty;
   const int x0 = tx * 16, y0 = ty * VT, z0 = tz * 4;
-  constexpr int cout = NT * 16;
-  const int ncb = cin >> 4;
+  // (three groups: the steps are faster with the stride as a number, 28.4 and
+  // 26.0 us at 64x32x32, 48 -> 48; the others with a constant)
+  const int cout = VT == 1 || NT == 3 ? ncout : NT * 16;
+  const int ncb = cin >> 4, c0 = VT == 1 ? blockIdx.y * (NT * 16) : 0;
   f4 acc[VT][NT];
 #pragma unroll
   for (int j = 0; j < VT; j++)
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[j][t] = f4{0.f, 0.f, 0.f, 0.f};
   const bf16x8 zero8 = {};
+  // chunk `it` (8 channels of a voxel) of input block cb
+  auto chunk = [&](int cb, int it) {
+    const int hv = it >> 1, half = it & 1;
+    const int hx = hv % HX, r = hv / HX, hy = r % HY, hz = r / HY;
+    const int gx = x0 - 1 + hx, gy = y0 - 1 + hy, gz = z0 - 1 + hz;
+    if (gx >= 0 && gx < d.W && gy >= 0 && gy < d.H && gz >= 0 && gz < d.D)
+      return *(const uint4 *)(x + (((long long)gz * d.H + gy) * d.W + gx) * cin + cb * 16 +
+                              half * 8);
+    return make_uint4(0u, 0u, 0u, 0u);
+  };
+  constexpr int NP = (2 * HV + 255) / 256;
+  uint4 v[NP];  // (AHEAD) the thread's chunks of the next input block
+  auto fetch = [&](int cb) {
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      const int it = threadIdx.x + 256 * k;
+      v[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (it < 2 * HV) v[k] = chunk(cb, it);
+    }
+  };
+  if (AHEAD) fetch(0);
   for (int cb = 0; cb < ncb; cb++) {
     __syncthreads();  // every wavefront is done with the previous block's tile
-    for (int it = threadIdx.x; it < 2 * HV; it += 256) {
-      const int hv = it >> 1, half = it & 1;
-      const int hx = hv % HX, r = hv / HX, hy = r % HY, hz = r / HY;
-      const int gx = x0 - 1 + hx, gy = y0 - 1 + hy, gz = z0 - 1 + hz;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (gx >= 0 && gx < d.W && gy >= 0 && gy < d.H && gz >= 0 && gz < d.D)
-        v = *(const uint4 *)(x + (((long long)gz * d.H + gy) * d.W + gx) * cin + cb * 16 +
-                             half * 8);
-      *(uint4 *)(tile + hv * 16 + half * 8) = v;
+    if (AHEAD) {
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        const int it = threadIdx.x + 256 * k;
+        if (it < 2 * HV) *(uint4 *)(tile + it * 8) = v[k];
+      }
+      if (cb + 1 < ncb) fetch(cb + 1);
+    } else {
+      for (int it = threadIdx.x; it < 2 * HV; it += 256) *(uint4 *)(tile + it * 8) = chunk(cb, it);
     }
     __syncthreads();
-    const uint16_t *wcb = wq + (long long)cb * 15 * cout * 32 + 8 * kg;
-#pragma unroll 3
+    const uint16_t *wcb = wq + ((long long)cb * 15 * cout + c0) * 32 + 8 * kg;
+#pragma unroll UN
     for (int q = 0; q < 15; q++) {
       const int dz = q / 5, t9 = 2 * (q % 5) + (kg >> 1);
       const bool real = t9 < 9;
@@ -141,7 +178,7 @@ __global__ __launch_bounds__(256) void k_conv3(const uint16_t *__restrict__ x, i
     if (zz >= d.D || yy >= d.H) continue;
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-      const int co = t * 16 + m;
+      const int co = c0 + t * 16 + m;
       const float bv = bias ? bias[co] : 0.f;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -1378,7 +1415,9 @@ int wm_unet_conv3(const uint16_t *x, int64_t cin, uint16_t *y, float *yf, int64_
       return 0;
     }
     // rows of 16 voxels per wavefront: 4 up to 64 output channels, 2 above;
-    // 1 where that leaves fewer than 256 blocks (the coarsest levels)
+    // 1, and 16 output channels per block, where that leaves fewer than 256
+    // blocks (the coarsest levels: 32x16x16 with 48 channels 128 -> 384
+    // blocks, 16x8x8 with 64 channels 32 -> 128)
     const int ntx = (int)((W + 15) / 16), nzb = (int)((D + 3) / 4);
     int vt = cout <= 64 ? 4 : 2;
     if ((long long)ntx * ((H + vt - 1) / vt) * nzb < 256) vt = 1;
@@ -1388,13 +1427,16 @@ int wm_unet_conv3(const uint16_t *x, int64_t cin, uint16_t *y, float *yf, int64_
     const dim3 g((unsigned)nblk), bl(256);
     auto run = [&](auto nt) {
       constexpr int NT = decltype(nt)::value;
-      if (vt == 1)
-        hipLaunchKernelGGL((k_conv3<NT, 1>), g, bl, 0, s, x, (int)cin, y, yf, d, wp, bias, sl, ntx,
-                           nty);
-      else
-        hipLaunchKernelGGL((k_conv3<NT, NT <= 4 ? 4 : 2>), g, bl, 0, s, x, (int)cin, y, yf, d, wp,
-                           bias, sl, ntx, nty);
+      hipLaunchKernelGGL((k_conv3<NT, NT <= 4 ? 4 : 2>), g, bl, 0, s, x, (int)cin, y, yf, d, wp,
+                         bias, sl, ntx, nty, (int)cout);
     };
+    if (vt == 1) {
+      WM_REQUIRE(cout <= 128, "wm_unet_conv3: cout > 128");
+      hipLaunchKernelGGL((k_conv3<1, 1>), dim3((unsigned)nblk, (unsigned)(cout / 16)), bl, 0, s, x,
+                         (int)cin, y, yf, d, wp, bias, sl, ntx, nty, (int)cout);
+      WM_LAUNCHED();
+      return 0;
+    }
     switch (cout / 16) {
       case 1: run(ic<1>()); break;
       case 2: run(ic<2>()); break;
