@@ -132,6 +132,25 @@ def test_boundary_conditions(device, bounds, lwd, lzd):
     np.testing.assert_array_equal(ug.cpu().numpy(), uo)
 
 
+@pytest.mark.parametrize("bounds", [(1,) * 6, (2,) * 6, (0, 1, 2, 2, 1, 0), (1, 0, 1, 1, 2, 2),
+                                    (0, 0, 1, 0, 0, 1)])
+@pytest.mark.parametrize("n", [(2, 2, 2), (1, 3, 2), (2, 1, 5), (3, 4, 1), (7, 66, 5)])
+def test_boundary_conditions_in_one_launch(device, n, bounds):
+    """Two or three axes at once against the oracle, axis after axis, at the
+    shortest axes (those of one cell go axis by axis): bitwise, corners
+    included."""
+    from warp_amd import _native as N
+    nx, ny, nz = n
+    u = np.random.default_rng(8).standard_normal((nz + 3, ny + 3, nx + 3))
+    ug = torch.from_numpy(u).to(device)
+    b = (C.c_int64 * 6)(*bounds)
+    N.call("wm_applyboundaryconditions3d", nx, ny, nz, ug.data_ptr(), b, 0, 0,
+           N.stream_of(device))
+    uo = u.copy()
+    O.applyboundaryconditions3d(uo, bounds, 0, 0)
+    np.testing.assert_array_equal(ug.cpu().numpy(), uo)
+
+
 def _c1_like(device, nx, ny, nz, precision="fp64", mgform=1, seed=5):
     """Pipe + annulus with a Gaussian beam's rho; returns (solver, oracle
     phi, oracle mgiters)."""

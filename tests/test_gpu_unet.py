@@ -57,6 +57,15 @@ def test_conv3_forward(device, cin, cout, dims):
     assert (got - ref).abs().max() <= 2e-5 * ref.abs().max() + 1e-6
 
 
+@pytest.mark.parametrize("cin,cout,dims", [(48, 64, (5, 9, 11)), (64, 128, (3, 5, 18)),
+                                           (80, 48, (4, 7, 33)), (64, 48, (40, 30, 60))])
+def test_conv3_channel_groups(device, cin, cout, dims):
+    """Grids with few blocks give a block 16 output channels (ragged tiles,
+    several input blocks), the last one four rows and three groups with the
+    next tile read ahead: against the same convolution in 64 bits."""
+    test_conv3_forward(device, cin, cout, dims)
+
+
 @pytest.mark.parametrize("cin,cout,dims", [(16, 16, (19, 22, 40)), (32, 16, (9, 13, 33)),
                                            (48, 16, (11, 9, 20)), (16, 16, (1, 3, 5)),
                                            (16, 32, (13, 17, 35)), (32, 32, (10, 9, 20))])
