@@ -132,9 +132,10 @@ def test_boundary_conditions(device, bounds, lwd, lzd):
     np.testing.assert_array_equal(ug.cpu().numpy(), uo)
 
 
-@pytest.mark.parametrize("bounds", [(1,) * 6, (2,) * 6, (0, 1, 2, 2, 1, 0), (1, 0, 1, 1, 2, 2),
-                                    (0, 0, 1, 0, 0, 1)])
-@pytest.mark.parametrize("n", [(2, 2, 2), (1, 3, 2), (2, 1, 5), (3, 4, 1), (7, 66, 5)])
+@pytest.mark.parametrize("n,bounds", [
+    (n, b) for n in ((2, 2, 2), (1, 3, 2), (2, 1, 5), (3, 4, 1), (7, 66, 5))
+    for b in ((1,) * 6, (2,) * 6, (0, 1, 2, 2, 1, 0), (1, 0, 1, 1, 2, 2), (0, 0, 1, 0, 0, 1))
+    if not any(n[a] == 1 and b[2 * a] == 2 for a in range(3))])  # (a periodic axis: two cells)
 def test_boundary_conditions_in_one_launch(device, n, bounds):
     """Two or three axes at once against the oracle, axis after axis, at the
     shortest axes (those of one cell go axis by axis): bitwise, corners
