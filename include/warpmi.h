@@ -206,9 +206,8 @@ int wm_setrho3d(double *rho, int64_t np, const double *xp, const double *yp,
  * Particles whose neighbours in the arrays are far apart on the mesh are
  * then ordered by tiles of the mesh before their charge is added, which
  * for unordered particles takes a fraction of the time.  The same sums in
- * another order.  work is zero-filled before its first call, belongs to one
- * mesh size, and is used by one call at a time (each leaves the counters it
- * starts from at zero again). */
+ * another order.  work holds nothing between calls; calls that may run at the
+ * same time (on two streams) take one each. */
 int64_t wm_setrho3d_worksize(int64_t np, int64_t nx, int64_t ny, int64_t nz);
 int wm_setrho3d_work(double *rho, int64_t np, const double *xp,
                      const double *yp, const double *zp, double zgrid,

@@ -117,6 +117,74 @@ def test_deposit_with_workspace(device, mesh, order, n):
     assert np.abs(r - ro).max() <= tol * np.abs(ro).max()
 
 
+def test_deposit_workspace_comes_as_it_is(device):
+    """A workspace that holds anything: all bits set, then what another count
+    of particles left.  1e-13 of the peak as above."""
+    from warp_amd import _native as N
+    q, w = 1.602176565e-19, 3.7e4
+    work = torch.full((N.lib().wm_setrho3d_worksize(300001, NX, NY, NZ),), 255,
+                      dtype=torch.uint8, device=device)
+    for n, seed in ((300001, 4), (262144, 5), (300001, 6)):
+        x, y, z = _beam(n, seed)
+        keep = [_t(v, device) for v in (x, y, z)]
+        rho = torch.zeros((NZ + 1, NY + 1, NX + 1), dtype=torch.float64, device=device)
+        N.call("wm_setrho3d_work", rho.data_ptr(), len(x), *[k.data_ptr() for k in keep], 0.0, q,
+               w, NX, NY, NZ, DX, DY, DZ, *LO, None, work.data_ptr(), work.numel(),
+               N.stream_of(device))
+        ro = np.zeros((NZ + 1, NY + 1, NX + 1))
+        O.setrho3d(ro, x, y, z, q, w, DX, DY, DZ, *LO)
+        assert np.abs(rho.cpu().numpy() - ro).max() <= 1e-13 * np.abs(ro).max()
+
+
+@pytest.mark.parametrize("grow", [False, True])
+def test_deposits_on_two_streams(device, grow):
+    """Groups deposited into one solver from two streams at once, and a group
+    that grows from one deposit to the next on a stream that is not the
+    solver's first: the sum of all of them (FP64 sums in another order:
+    1e-13 of the peak)."""
+    from warp_amd.multigrid import MultiGrid3D
+    s = MultiGrid3D(nx=NX, ny=NY, nz=NZ, xmmin=LO[0], xmmax=-LO[0], ymmin=LO[1], ymmax=-LO[1],
+                    zmmin=LO[2], zmmax=LO[2] + NZ * DZ, bounds=[0] * 6, device=device,
+                    mgverbose=-1)
+    q, w = 1.602176565e-19, 3.7e4
+    streams = [torch.cuda.Stream(device), torch.cuda.Stream(device)]
+    sizes = [(300000, 300000)] * 3 if not grow else [(300000, 300000 + 50000 * k)
+                                                     for k in range(6)]
+    beams = [[_beam(n, 10 + 2 * k + i) for i, n in enumerate(p)] for k, p in enumerate(sizes)]
+    dev = [[[_t(v, device) for v in b] for b in p] for p in beams]
+    s.zerosourcep()
+    torch.cuda.synchronize()
+    for p in dev:
+        for st, b in zip(streams, p):
+            with torch.cuda.stream(st):
+                s.setsourcepatposition(*b, 0., q, w)
+    torch.cuda.synchronize()
+    ro = np.zeros((NZ + 1, NY + 1, NX + 1))
+    for b in sum(beams, []):
+        O.setrho3d(ro, *b, q, w, s.dx, s.dy, s.dz, *LO)
+    assert np.abs(s.rho.cpu().numpy() - ro).max() <= 1e-13 * np.abs(ro).max()
+
+
+def test_deposit_where_the_workspace_does_not_fit(device, monkeypatch):
+    """No memory for the workspace: the deposit does without it."""
+    from warp_amd.multigrid import MultiGrid3D
+    s = MultiGrid3D(nx=NX, ny=NY, nz=NZ, xmmin=LO[0], xmmax=-LO[0], ymmin=LO[1], ymmax=-LO[1],
+                    zmmin=LO[2], zmmax=LO[2] + NZ * DZ, bounds=[0] * 6, device=device,
+                    mgverbose=-1)
+    x, y, z = _beam(300000, 3)
+    keep = [_t(v, device) for v in (x, y, z)]
+
+    def none(*a, **k):
+        raise torch.cuda.OutOfMemoryError("none left")
+
+    monkeypatch.setattr(torch, "empty", none)
+    s.setsourcepatposition(*keep, 0., 1., 2.)
+    monkeypatch.undo()
+    ro = np.zeros((NZ + 1, NY + 1, NX + 1))
+    O.setrho3d(ro, x, y, z, 1., 2., s.dx, s.dy, s.dz, *LO)
+    assert np.abs(s.rho.cpu().numpy() - ro).max() <= 1e-13 * np.abs(ro).max()
+
+
 def test_deposit_worksize_limits():
     """No workspace for meshes of more tiles than a block can count."""
     from warp_amd import _native as N

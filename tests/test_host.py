@@ -349,3 +349,36 @@ def test_special_step_cadence():
         assert special_step(False)[0]
     finally:
         top.it, top.time, top.allspecl = saved
+
+
+@pytest.mark.parametrize("sort", [False, True])
+def test_deposits_in_flight_share_no_workspace(sort, monkeypatch):
+    """A deposit that begins while another into the same solver is still
+    running (another stream or thread) has a workspace of its own, of the
+    same, a smaller or a larger group."""
+    import torch
+    from warp_amd import _native as N
+    from warp_amd.multigrid import MultiGrid3D
+    s = MultiGrid3D.__new__(MultiGrid3D)
+    s.__dict__.update(device=torch.device("cpu"), sorted_deposit=sort, nx=64, ny=64, nz=64,
+                      dx=1., dy=1., dz=1., xmmin=0., ymmin=0., zmmin=0., _rho=torch.zeros(1))
+    sizes = [300000, 300000, 262144, 400000]
+    live = []
+
+    def call(name, *args):
+        base, need = (args[-2], N.lib().wm_setrho3d_sorted_worksize(args[1], 64, 64, 64)) \
+            if sort else args[-3:-1]
+        assert need > 0
+        assert all(base + need <= b or b + n <= base for b, n in live)
+        live.append((base, need))
+        if len(live) < len(sizes):  # the next one begins before this one ends
+            deposit(sizes[len(live)])
+        live.pop()
+
+    def deposit(n):
+        x = torch.zeros(n, dtype=torch.float64)
+        s.setsourcepatposition(x, x, x, 0., 1., 1.)
+
+    monkeypatch.setattr(N, "call", call)
+    monkeypatch.setattr(N, "stream_of", lambda device: None)
+    deposit(sizes[0])

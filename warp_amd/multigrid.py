@@ -73,8 +73,6 @@ class MultiGrid3D(FieldSolver):
         self._rho = torch.zeros((self.nz + 1, self.ny + 1, self.nx + 1), dtype=torch.float64,
                                 device=self.device)
         self._selfe = None
-        self._work = None          # of the sorted deposit
-        self._binwork = None       # of the deposit (counters zero between calls)
         self._nlost = None
         self._cf = None            # conductor field data for f3d.lcorrectede
         self._cf_key = None
@@ -302,26 +300,31 @@ class MultiGrid3D(FieldSolver):
         self.setsourcepatposition(x, y, z, zgrid, q, w)
 
     def setsourcepatposition(self, x, y, z, zgrid, q, w):
-        """setrho3d (w3d.F:7199-7301) on the GPU."""
+        """setrho3d (w3d.F:7199-7301) on the GPU.  The workspace is the
+        call's own, from the current stream's memory pool and back to it:
+        deposits of several streams or threads into one solver (whose sums
+        are atomic) share nothing else, and what frees it is ordered behind
+        the kernels that use it."""
         n = int(x.numel())
         if n == 0:
             return
         s = N.stream_of(self.device)
         if self.sorted_deposit:
             need = N.lib().wm_setrho3d_sorted_worksize(n, self.nx, self.ny, self.nz)
-            if self._work is None or self._work.numel() < need:
-                self._work = torch.empty(int(need), dtype=torch.uint8, device=self.device)
+            work = torch.empty(int(need), dtype=torch.uint8, device=self.device)
             N.call("wm_setrho3d_sorted", self._rho.data_ptr(), n, x.data_ptr(), y.data_ptr(),
                    z.data_ptr(), zgrid, q, w, self.nx, self.ny, self.nz, self.dx, self.dy,
-                   self.dz, self.xmmin, self.ymmin, self.zmmin, self._work.data_ptr(), s)
+                   self.dz, self.xmmin, self.ymmin, self.zmmin, work.data_ptr(), s)
         else:
             need = N.lib().wm_setrho3d_worksize(n, self.nx, self.ny, self.nz)
-            if need and (self._binwork is None or self._binwork.numel() < need):
-                self._binwork = torch.zeros(need, dtype=torch.uint8, device=self.device)
+            try:
+                work = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
+            except torch.cuda.OutOfMemoryError:
+                work, need = None, 0  # the deposit does without
             N.call("wm_setrho3d_work", self._rho.data_ptr(), n, x.data_ptr(), y.data_ptr(),
                    z.data_ptr(), zgrid, q, w, self.nx, self.ny, self.nz, self.dx, self.dy,
                    self.dz, self.xmmin, self.ymmin, self.zmmin, None,
-                   self._binwork.data_ptr() if need else None, need, s)
+                   work.data_ptr() if need else None, need, s)
 
     def finalizesourcep(self):
         if self.sourcepfinalized:
