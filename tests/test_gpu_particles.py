@@ -1,6 +1,7 @@
 """GPU parity of the particle kernels (deposit, gather, push, grid E)
 against the FP64 oracle."""
 import ctypes as C
+import math
 
 import numpy as np
 import pytest
@@ -73,14 +74,17 @@ def test_deposit_matches_oracle(device, order):
 
 @pytest.mark.parametrize("mesh", [(NX, NY, NZ), (33, 16, 47), (5, 70, 31), (250, 255, 510)])
 @pytest.mark.parametrize("order", ["random", "cell_ordered", "drifted", "clumped"])
-@pytest.mark.parametrize("n", [262143, 262144, 300001])
+@pytest.mark.parametrize("n", [-1, 0, 262144, 300001])
 def test_deposit_with_workspace(device, mesh, order, n):
     """setrho3d with a workspace: boxes, boxes plane by plane and the binned
     particles, on meshes whose last tiles of 16 cells are full, cut or one
-    cell thin, with particles outside; below 262144 particles there is
-    no workspace.  FP64 sums in another order: 1e-13 of the peak."""
+    cell thin, with particles outside; at the fewest particles that take a
+    workspace (0), and one less.  FP64 sums in another order: 1e-13 of the
+    peak."""
     from warp_amd import _native as N
     nx, ny, nz = mesh
+    least = 32768 + 16 * math.prod(-(-m // 16) for m in mesh)
+    n = n if n > 0 else least + n
     hi = (-LO[0], -LO[1], 0.08)
     d = [(hi[k] - LO[k]) / m for k, m in enumerate(mesh)]
     x, y, z = [v[:n] for v in _beam(n + 5000, 3)]
@@ -97,7 +101,7 @@ def test_deposit_with_workspace(device, mesh, order, n):
     for k, v in enumerate((x, y, z)):
         inside &= (v >= LO[k]) & ((v - LO[k]) * (1. / d[k]) < mesh[k])
     need = N.lib().wm_setrho3d_worksize(n, *mesh)
-    assert (need > 0) == (n >= 262144)
+    assert (need > 0) == (n >= least)
     work = torch.zeros(need, dtype=torch.uint8, device=device)
     keep = [_t(v, device) for v in (x, y, z)]
     ns = C.c_int64(-1)

@@ -382,3 +382,28 @@ def test_deposits_in_flight_share_no_workspace(sort, monkeypatch):
     monkeypatch.setattr(N, "call", call)
     monkeypatch.setattr(N, "stream_of", lambda device: None)
     deposit(sizes[0])
+
+
+def test_few_unordered_particles_are_binned():
+    """Which deposits take a workspace: unordered ones from the library's
+    limit on (0.1M on 64^3, far below 262144), which grows with the mesh's
+    tiles; ordered ones of fewer than 262144 only where they are sparse; and
+    what a group says of its order."""
+    import torch
+    from warp_amd import _native as N
+    from warp_amd.multigrid import MultiGrid3D
+    from warp_amd.particles import ParticleGroup
+    f = N.lib().wm_setrho3d_worksize
+    for mesh, tiles in (((64, 64, 64), 64), ((128, 128, 256), 1024), ((256, 256, 512), 8192),
+                        ((17, 1, 1), 2)):
+        assert f(32768 + 16 * tiles, *mesh) > 0 and f(32767 + 16 * tiles, *mesh) == 0
+    s = MultiGrid3D.__new__(MultiGrid3D)
+    s.nx = s.ny = s.nz = 64
+    assert s._binned(32767, True) and not s._binned(32768, True) and s._binned(32768, False)
+    assert not s._binned(262143, True) and s._binned(262144, True)
+    pg = ParticleGroup("cpu")
+    pg.addspecies(1., 1., 1.)
+    pg.ordered = True
+    v = torch.zeros(3, dtype=torch.float64)
+    pg.addparticles(0, *[v] * 6)
+    assert not pg.ordered

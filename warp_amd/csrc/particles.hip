@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256) void k_setrho(double *__restrict__ rho, long l
 // and the LDS atomics: 4M unordered particles on 128x128x256 take 265 us where
 // the scattered atomics took 1910 us, 16M 0.92 ms against 7.6, 32M on
 // 256x256x512 2.4 ms against 10.9.  All sizes come from the device-side list, so
-// the two launches return at once when it is empty (4 us).
+// the launches return at once when it is empty (5 us, k_bin_clear's included).
 constexpr int BIN_NODES = (BIN_T + 1) * (BIN_T + 1) * (BIN_T + 1);
 constexpr int BIN_MAXTILES = 4 * DEP_BOX;  // 16-bit counters of one k_setrho block
 constexpr int BIN_THREADS = 1024;
@@ -323,12 +323,14 @@ constexpr int BIN_GROUP = 8;               // listed blocks taken at a time at m
                                            // particle of each per thread
 constexpr int BIN_PIECE = 4096;            // particles per piece of a tile, at least
 constexpr int BIN_PIECES = 2048;           // pieces beyond one per tile, at most
-// Fewer particles than this take no workspace: unordered, 100,000 take 54 us
-// by scattered atomics and 27 us binned, 200,000 (on 64^3) 175 and 38 us, but
-// ordered, as a step driver keeps them, they need no list, and the two more
-// launches cost such a short step 1% (5.47 -> 5.53 ms per five steps on 64^3
-// with 200,000).
-constexpr int BIN_MIN = 262144;
+// Fewer particles than this take no workspace.  Binned, unordered particles
+// cost three launches' latency and every block's look at all tiles' counts,
+// scattered their atomics; the line follows the tiles (us scattered / binned):
+//   12 tiles (24x24x32):        16,000 20/27   32,000 31/27   100,000 92/30
+//   64 (64x64x64):              16,000 19/23   32,000 30/28   100,000 82/33
+//   1024 (128x128x256):         32,000 22/23   65,536 38/25   200,000 101/37
+//   8192 (256x256x512):        100,000 40/53  200,000 75/67   500,000 179/104
+inline int64_t bin_min(int64_t ntiles) { return 32768 + 16 * ntiles; }
 static_assert(DEP_PART == BIN_THREADS, "one particle of a listed block per thread");
 
 // Exclusive sum of v over the block's BIN_THREADS threads; total to all.
@@ -998,7 +1000,9 @@ struct BinLayout {
 static BinLayout bin_layout(int64_t np, int64_t nx, int64_t ny, int64_t nz) {
   BinLayout w{};
   const int64_t ntx = cdiv(nx, BIN_T), nty = cdiv(ny, BIN_T), ntz = cdiv(nz, BIN_T);
-  if (ntx * nty * ntz > BIN_MAXTILES || np >= (1ll << 31) || np < BIN_MIN) return w;
+  if (ntx * nty * ntz > BIN_MAXTILES || np >= (1ll << 31) ||
+      np < bin_min(ntx * nty * ntz))
+    return w;
   w.ntx = (int)ntx;
   w.nty = (int)nty;
   w.ntiles = (int)(ntx * nty * ntz);

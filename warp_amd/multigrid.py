@@ -297,14 +297,28 @@ class MultiGrid3D(FieldSolver):
         x, y, z = pgroup.xp[sl], pgroup.yp[sl], pgroup.zp[sl]
         q = pgroup.sq[js]
         w = pgroup.sw[js] * pgroup.dtscale[js]
-        self.setsourcepatposition(x, y, z, zgrid, q, w)
+        self.setsourcepatposition(x, y, z, zgrid, q, w,
+                                  ordered=getattr(pgroup, "ordered", False))
 
-    def setsourcepatposition(self, x, y, z, zgrid, q, w):
+    # Ordered particles need no bins where they are dense enough that the
+    # nodes which a block of them touches fit its box: from a particle per
+    # eight cells on.  On 64^3 cells 100,000 of them take 17 us without the
+    # workspace and 22 with it, 262,144 8 and 14 (five steps with 200,000 5.47
+    # and 5.53 ms), on 128x128x256 65,536 39 and 26, 500,000 62 and 39.  From
+    # 262,144 on what they have drifted matters more than the launches: 4M on
+    # 128x128x256 147 and 73 us.
+    ORDERED_MIN = 262144
+
+    def _binned(self, n, ordered):
+        return not (ordered and n < self.ORDERED_MIN and 8 * n >= self.nx * self.ny * self.nz)
+
+    def setsourcepatposition(self, x, y, z, zgrid, q, w, ordered=False):
         """setrho3d (w3d.F:7199-7301) on the GPU.  The workspace is the
         call's own, from the current stream's memory pool and back to it:
         deposits of several streams or threads into one solver (whose sums
         are atomic) share nothing else, and what frees it is ordered behind
-        the kernels that use it."""
+        the kernels that use it.  ordered: the particles come by mesh cell
+        or nearly so (a matter of speed alone)."""
         n = int(x.numel())
         if n == 0:
             return
@@ -316,7 +330,8 @@ class MultiGrid3D(FieldSolver):
                    z.data_ptr(), zgrid, q, w, self.nx, self.ny, self.nz, self.dx, self.dy,
                    self.dz, self.xmmin, self.ymmin, self.zmmin, work.data_ptr(), s)
         else:
-            need = N.lib().wm_setrho3d_worksize(n, self.nx, self.ny, self.nz)
+            need = (N.lib().wm_setrho3d_worksize(n, self.nx, self.ny, self.nz)
+                    if self._binned(n, ordered) else 0)
             try:
                 work = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
             except torch.cuda.OutOfMemoryError:

@@ -25,6 +25,9 @@ class ParticleGroup:
         self.sq, self.sm, self.sw, self.dtscale = [], [], [], []
         self.ins, self.nps = [], []  # 1-based start, count (as the reference)
         self.ndts = []
+        # the particles come by mesh cell (particlesortxyzwithcopy) but for
+        # what they have moved since: what a deposit may do about their order
+        self.ordered = False
 
     @property
     def ns(self):
@@ -74,6 +77,7 @@ class ParticleGroup:
             v = torch.as_tensor(cols[c], dtype=self.dtype, device=self.device).reshape(-1)
             setattr(self, c, torch.cat([getattr(self, c), v]))
         self.nps[js] += n
+        self.ordered = False
 
     def species_slice(self, js):
         i = self.ins[js] - 1
@@ -168,6 +172,7 @@ def particlesortxyzwithcopy(pgroup, dx, dy, dz, xmmin, ymmin, zmmin, nx, ny, nz)
     # slots outside every species' live block hold nothing: left unset
     for c in pgroup.COLUMNS:
         setattr(pgroup, c, new[c])
+    pgroup.ordered = True
 
 
 def gaussian_weight(current, sigmaz, vz, charge, npart):
