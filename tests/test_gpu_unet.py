@@ -230,17 +230,26 @@ def test_conv3_weight_gradient_shapes(device, cin, cout, dims):
     assert (db.cpu().to(torch.float64) - b.grad).abs().max() <= 1e-5 * b.grad.abs().max()
 
 
-@pytest.mark.parametrize("cin,cout,dims", [(16, 16, (4, 8, 16)), (48, 16, (5, 9, 11)),
-                                           (16, 64, (2, 3, 240)), (32, 48, (3, 130, 1)),
-                                           (64, 32, (1, 1, 17)), (16, 32, (40, 20, 24))])
-def test_conv3_weight_gradient_forms(device, cin, cout, dims):
+@pytest.mark.parametrize("cin,cout,dims,form", [
+    (16, 16, (4, 8, 16), "rows"), (48, 16, (5, 9, 11), "rows"), (32, 48, (3, 130, 1), "rows"),
+    (64, 32, (1, 1, 17), "rows"), (16, 32, (40, 20, 24), "rows"),
+    # rings of more than 64 KB, up to the most that two blocks share
+    (16, 64, (2, 3, 41), "rows"), (16, 64, (2, 3, 42), "rows above 64 KB"),
+    (16, 64, (2, 5, 126), "rows above 64 KB"), (16, 16, (3, 2, 200), "rows above 64 KB"),
+    (32, 32, (2, 2, 210), "rows above 64 KB"),
+    (16, 64, (2, 3, 127), "tiles"), (16, 64, (2, 3, 240), "tiles")])
+def test_conv3_weight_gradient_forms(device, cin, cout, dims, form):
     """The row form of the weight gradient against the tile form, which takes
-    over where an operand is not 16-byte aligned: the same sums in the same
-    order, so dW has the same bits.  Grids of one chunk and of many, rows
-    shorter and longer than a step, and one whose rings need more than 64 KB;
-    an infinite input value reaches the same taps in both."""
+    over where an operand is not 16-byte aligned or a row too long: the same
+    sums in the same order, so dW has the same bits.  Grids of one chunk and
+    of many, rows shorter and longer than a step, rings on either side of 64
+    KB and of the 80 KB that are too many; an infinite input value reaches the
+    same taps in both."""
     from warp_amd import _native as N
     D, H, W = dims
+    # three rings of two rows and two steps of 128 voxels, two steps of g
+    lds = 2 * (16 + 3 * (2 * W + 2 + 256) * 16 + 2 * 128 * cout)
+    assert form == ("tiles" if lds > 81920 else "rows above 64 KB" if lds > 65536 else "rows")
     g = torch.Generator().manual_seed(cin + cout + W)
     n = D * H * W
     x = (torch.randn(n * cin, generator=g)).to(torch.bfloat16)
