@@ -129,8 +129,8 @@ int wm_mg3d_last_reused(const wm_mg3d *h, int64_t *reused);
  * WARPMI_TAIL_LDS (bytes; 0 switches the single launch off) caps the LDS
  * budget that decides the level, read when the solver is created. */
 int wm_mg3d_tail_start(const wm_mg3d *h, int64_t *level);
-/* Bit l of *levels is set when the solver's last preparation let level l's
- * V-cycle run as one launch down and one up. */
+/* Bit l of *levels is set when the V-cycles of the solver's last solve ran
+ * level l as one launch down and one up. */
 int wm_mg3d_leg_levels(const wm_mg3d *h, int64_t *levels);
 
 /* Form of the SOR passes (sorpass3d, f3d_mgrid.F:1949-2093): 0 = two

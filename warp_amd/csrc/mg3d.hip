@@ -345,6 +345,7 @@ struct wm_mg3d {
   // (WARPMI_LEG_NODES; 0: none), see leg_limit
   long long leg_nodes = getenv("WARPMI_LEG_NODES") ? atoll(getenv("WARPMI_LEG_NODES")) : LEG_NODES;
   bool tail_used = false;  // the last solve was FP64 and ran the tail
+  int64_t legs_used = 0;   // bit l: the last solve's V-cycles ran level l by legs
   size_t tail_lds = 0;
   int ncu = 256;                 // compute units of the device
   size_t lds_per_cu = 160 * 1024;
@@ -2179,8 +2180,15 @@ static long long leg_limit(const wm_mg3d *h, const Level &L) {
   return L.hasmask ? 2 * h->leg_nodes : h->leg_nodes;
 }
 
+// The levels a V-cycle with the parameters P enters: up to the tail's.
+static int entered_levels(const wm_mg3d *h, const Params &P) {
+  const int n = (int)h->lv.size();
+  return h->tail.on && tail_applies(h, h->tail.start, P) ? h->tail.start : n;
+}
+
 static void prepare_legs(wm_mg3d *h, const Params &P) {
-  for (int l = 1; l + 1 < (int)h->lv.size(); l++) {
+  const int end = std::min(entered_levels(h, P), (int)h->lv.size() - 1);
+  for (int l = 1; l < end; l++) {
     Level &L = *h->lv[l];
     const long long nodes = (long long)(L.nx + 1) * (L.ny + 1) * (L.nz + 1);
     RecKey key;
@@ -2756,6 +2764,9 @@ int wm_mg3d_solve(wm_mg3d *h, double *phi, double *rho, double mgparam, int64_t 
     prepare_tail(h, P);
     prepare_legs(h, P);
     h->tail_used = h->tail.on && prec == WM_PREC_FP64 && mgmaxiters > 0;
+    h->legs_used = 0;
+    for (int l = 1; l < std::min(entered_levels(h, P), 63) && mgmaxiters > 0; l++)
+      if (leg_level(h, l, P)) h->legs_used |= (int64_t)1 << l;
     // Inputs.
     WM_HIP(hipEventRecord(h->ev_in, us));
     WM_HIP(hipStreamWaitEvent(s, h->ev_in, 0));
@@ -3023,9 +3034,7 @@ int wm_mg3d_tail_start(const wm_mg3d *h, int64_t *level) {
 int wm_mg3d_leg_levels(const wm_mg3d *h, int64_t *levels) {
   WM_ENTRY({
     WM_REQUIRE(h && levels, "wm_mg3d_leg_levels: NULL argument");
-    *levels = 0;
-    for (size_t l = 1; l < h->lv.size() && l < 63; l++)
-      if (h->lv[l]->leg_ok) *levels |= 1ll << l;
+    *levels = h->legs_used;
   });
 }
 

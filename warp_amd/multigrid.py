@@ -433,8 +433,8 @@ class MultiGrid3D(FieldSolver):
         return int(r.value)
 
     def leg_levels(self):
-        """The coarse levels whose V-cycle runs as one launch down and one
-        up, as far as the last solve's parameters allow."""
+        """The coarse levels that the last solve's V-cycles ran as one launch
+        down and one up each."""
         r = C.c_int64(0)
         N.call("wm_mg3d_leg_levels", self._h, C.byref(r))
         return [l for l in range(63) if r.value >> l & 1]
