@@ -190,17 +190,27 @@ struct CondDev {
 };
 
 // The tiles of one leg (mg3d_leg.h) on a level: the axes (their tables are
-// the level's), the records of the tiles' windows, the launch.
+// the level's) and the launch, the mesh's for good, and the records of the
+// tiles' windows, one setting's.
 struct LegTiles {
+  int made = -1;  // whether the mesh allows the leg (-1: not looked at yet)
   LegAxis a[3];
   DevBuf<LegTile> tile[3];
-  DevBuf<uint32_t> first;
-  DevBuf<LegRec> rec;
   int blocks = 0, values = 0;  // values: LDS values of a phi-sized window
   size_t lds(size_t value) const {
     return value * (2 * (size_t)values + coarse);
   }
   int coarse = 0;  // coarse phi values (up)
+  // per axis and node: its tiles and its coordinates in their windows,
+  // in[k][at[k][i]] .. in[k][at[k][i + 1]]
+  struct In {
+    int tile, at;
+  };
+  std::vector<int> at[3];
+  std::vector<In> in[3];
+  long long nrec = 0;
+  DevBuf<uint32_t> first;
+  DevBuf<LegRec> rec;
 };
 
 struct Level {
@@ -242,10 +252,12 @@ struct Level {
   // an active subgrid record sits on an interior (pinned) point, so the
   // pin after each half sweep is not a no-op
   bool sub_on_interior = false;
-  // faces_of (-1: not looked at yet), the interior points and, per element, the
-  // sides across which it reads one before the pin
+  // (coarse levels) the interior points and the active subgrid points on the
+  // host, these as build_mask left them, in the records' order
+  std::vector<int> int_h, rec_h[2];
+  // faces_of (-1: not looked at yet) and, per element, the sides across which
+  // it reads an interior point before the pin
   int faces = -1;
-  std::vector<int> int_h;
   std::vector<uint8_t> raw_h;
   std::vector<int> subpos_h[2];
   std::vector<double> subdels_h[2], subvolt_h[2];
@@ -678,8 +690,13 @@ static void build_mask(wm_mg3d *h, Level &L, int level, const Params &P) {
   std::vector<int> ipos;
   bool any = false;
   if (L.nint > 0) {
-    std::vector<int> hp(3 * L.nint);
-    WM_HIP(hipMemcpy(hp.data(), L.int_pos.p, sizeof(int) * hp.size(), hipMemcpyDeviceToHost));
+    std::vector<int> down;
+    if (level == 0) {
+      down.resize(3 * L.nint);
+      WM_HIP(hipMemcpy(down.data(), L.int_pos.p, sizeof(int) * down.size(),
+                       hipMemcpyDeviceToHost));
+    }
+    const std::vector<int> &hp = level == 0 ? down : L.int_h;
     for (int i = 0; i < L.nint; i++) setbit(hp[3 * i], hp[3 * i + 1], hp[3 * i + 2]);
     any = true;
     L.imask.upload(m);
@@ -687,6 +704,8 @@ static void build_mask(wm_mg3d *h, Level &L, int level, const Params &P) {
     L.imask.release();
   }
   L.sub_on_interior = false;
+  L.rec_h[0].clear();
+  L.rec_h[1].clear();
   if (P.lcnd) {
     for (int p = 0; p < 2; p++) {
       SubHost sh = build_records(L, level, p, h->bounds, P.mgparam, 1, P.icnd, false, false);
@@ -696,6 +715,7 @@ static void build_mask(wm_mg3d *h, Level &L, int level, const Params &P) {
         setbit(sh.pos[3 * i], sh.pos[3 * i + 1], sh.pos[3 * i + 2]);
         any = true;
       }
+      if (level > 0) L.rec_h[p].swap(sh.pos);
     }
   }
   if (any) L.mask.upload(m);
@@ -1579,6 +1599,7 @@ enum {
   FACES_UNEVEN = 2,  // an interior point of plane n whose image on plane 0 is not
   FACES_NO = 4,      // the form does not give the reference's values
 };
+// (a coarse level)
 static int faces_of(const wm_mg3d *h, Level &L) {
   if (L.faces >= 0) return L.faces;
   const int n[3] = {L.nx, L.ny, L.nz};
@@ -1589,10 +1610,6 @@ static int faces_of(const wm_mg3d *h, Level &L) {
     if (h->bounds[2 * a] == 2 && n[a] % 2) f |= FACES_NO;  // the colours do not meet
   }
   if (!f && face && L.nint > 0) {
-    // (downloads the points: once per conductor set)
-    L.int_h.resize(3 * L.nint);
-    WM_HIP(hipMemcpy(L.int_h.data(), L.int_pos.p, sizeof(int) * L.int_h.size(),
-                     hipMemcpyDeviceToHost));
     L.raw_h.assign((size_t)(2 * L.g.cs), 0);
     std::vector<bool> at((size_t)(L.nx + 1) * (L.ny + 1) * (L.nz + 1), false);
     auto node = [&](const int *q) {
@@ -2011,15 +2028,13 @@ static bool leg_level(const wm_mg3d *h, int level, const Params &P) {
          P.up == 1 && !fused_ok(h, L, level, P) && !tail_applies(h, level, P);
 }
 
-// The tiles of one leg: windows, launch and the records in each window.
-static bool build_leg(wm_mg3d *h, Level &L, const Level &Lc, LegTiles &D, bool up,
-                      const SubHost *recs) {
+// The tiles of one leg: windows and launch.
+static bool make_tiles(const wm_mg3d *h, const Level &L, const Level &Lc, LegTiles &D, bool up) {
   const int n[3] = {L.nx, L.ny, L.nz}, nc[3] = {Lc.nx, Lc.ny, Lc.nz};
   const int *b = h->bounds;
   // fine nodes of a tile, smaller where the level would give few blocks
   static const int shapes[3][3] = {{16, 8, 8}, {8, 8, 8}, {8, 4, 4}};
   static const int least[3] = {256, 64, 0};
-  static const int shape_env = getenv("WARPMI_LEG_SHAPE") ? atoi(getenv("WARPMI_LEG_SHAPE")) : -1;
   struct Win { int w0, w1; };
   std::vector<Win> win[3];
   std::vector<LegTile> tiles[3];
@@ -2110,55 +2125,60 @@ static bool build_leg(wm_mg3d *h, Level &L, const Level &Lc, LegTiles &D, bool u
     if (blocks >= (1ll << 30)) return false;
     D.blocks = (int)blocks;
     fits = fits && D.lds(8) <= 60000;
-    if (fits && (shape_env >= 0 ? q >= shape_env : blocks >= least[q])) break;
+    if (fits && blocks >= least[q]) break;
     if (q == 2 && !fits) return false;
   }
   for (int k = 0; k < 3; k++) {
     D.tile[k].upload(tiles[k]);
     D.a[k].tile = D.tile[k].p;
   }
-  // tiles and local coordinates of every node, per axis
-  std::vector<std::vector<std::pair<int, int>>> in[3];
   for (int k = 0; k < 3; k++) {
-    in[k].resize(n[k] + 1);
+    auto node = [&](int i) { return b[2 * k] == 2 ? (i % n[k] + n[k]) % n[k] : i; };
+    std::vector<int> &at = D.at[k];
+    at.assign(n[k] + 2, 0);
+    for (const Win &w : win[k])
+      for (int i = w.w0; i <= w.w1; i++) at[node(i) + 1]++;
+    for (int i = 0; i <= n[k]; i++) at[i + 1] += at[i];
+    D.in[k].resize(at[n[k] + 1]);
+    std::vector<int> to(at.begin(), at.end() - 1);
     for (int t = 0; t < D.a[k].nt; t++)
-      for (int i = win[k][t].w0; i <= win[k][t].w1; i++) {
-        const int u = b[2 * k] == 2 ? (i % n[k] + n[k]) % n[k] : i;
-        in[k][u].push_back({t, i - win[k][t].w0});
-      }
-  }
-  std::vector<std::vector<LegRec>> lists;
-  long long total = 0;
-  if (recs[0].n() + recs[1].n() > 0) {
-    lists.resize(D.blocks);
-    for (int p = 0; p < 2; p++)
-      for (int i = 0; i < recs[p].n(); i++) {
-        const int *q = &recs[p].pos[3 * i];
-        const uint32_t raw = L.raw_h.empty() ? 0u : L.raw_h[rb_index(L.g, q[0], q[1], q[2])];
-        for (auto &z : in[2][q[2]])
-          for (auto &y : in[1][q[1]])
-            for (auto &x : in[0][q[0]]) {
-              lists[x.first + D.a[0].nt * (y.first + D.a[1].nt * z.first)].push_back(
-                  LegRec{(uint32_t)(x.second | y.second << 8 | z.second << 16) | raw << 24,
-                         (uint32_t)p << 31 | (uint32_t)i});
-              total++;
-            }
-      }
-  }
-  std::vector<uint32_t> first(1, 0u);
-  std::vector<LegRec> flat;
-  flat.reserve((size_t)total);
-  for (auto &l : lists) {
-    flat.insert(flat.end(), l.begin(), l.end());
-    first.push_back((uint32_t)flat.size());
-  }
-  D.rec.release();
-  D.first.release();
-  if (total > 0) {
-    D.first.upload(first);
-    D.rec.upload(flat);
+      for (int i = win[k][t].w0; i <= win[k][t].w1; i++)
+        D.in[k][to[node(i)]++] = LegTiles::In{t, i - win[k][t].w0};
   }
   return true;
+}
+
+// The records of each tile's window: both colours' lists, which become one
+// list a tile (counted first, then written).
+static void place_records(const Level &L, LegTiles &D) {
+  std::vector<uint32_t> first((size_t)D.blocks + 1, 0u);
+  std::vector<LegRec> rec;
+  auto each = [&](auto &&put) {
+    for (int p = 0; p < 2; p++)
+      for (int i = 0; 3 * (size_t)i < L.rec_h[p].size(); i++) {
+        const int *q = &L.rec_h[p][3 * i];
+        for (int z = D.at[2][q[2]]; z < D.at[2][q[2] + 1]; z++)
+          for (int y = D.at[1][q[1]]; y < D.at[1][q[1] + 1]; y++)
+            for (int x = D.at[0][q[0]]; x < D.at[0][q[0] + 1]; x++) {
+              const LegTiles::In &X = D.in[0][x], &Y = D.in[1][y], &Z = D.in[2][z];
+              put((size_t)(X.tile + D.a[0].nt * (Y.tile + D.a[1].nt * Z.tile)), p, i, q,
+                  (uint32_t)(X.at | Y.at << 8 | Z.at << 16));
+            }
+      }
+  };
+  each([&](size_t t, int, int, const int *, uint32_t) { first[t + 1]++; });
+  for (int t = 0; t < D.blocks; t++) first[t + 1] += first[t];
+  D.nrec = first[D.blocks];
+  if (D.nrec == 0) return;
+  rec.resize((size_t)D.nrec);
+  std::vector<uint32_t> to(first.begin(), first.end() - 1);
+  each([&](size_t t, int p, int i, const int *q, uint32_t at) {
+    const uint32_t raw = L.raw_h.empty() ? 0u : L.raw_h[rb_index(L.g, q[0], q[1], q[2])];
+    rec[to[t]++] = LegRec{at | raw << 24, (uint32_t)p << 31 | (uint32_t)i};
+  });
+  D.first.upload(first);
+  if (D.rec.n < rec.size()) D.rec.alloc(rec.size());
+  WM_HIP(hipMemcpy(D.rec.p, rec.data(), sizeof(LegRec) * rec.size(), hipMemcpyHostToDevice));
 }
 
 // Legs need: one pin at most per pass that does something a tile can do for
@@ -2199,37 +2219,34 @@ static void prepare_legs(wm_mg3d *h, const Params &P) {
     L.leg_ok = false;
     if (!L.coarser || nodes > leg_limit(h, L) || L.sub_on_interior || (P.icnd == 2 && L.neumann))
       continue;
-    SubHost sor[2];
-    bool ok = true;
-    for (int p = 0; p < 2 && P.lcnd; p++) {
-      sor[p] = build_records(L, l, p, h->bounds, P.mgparam, P.mgform, P.icnd, false, false);
-      const SubHost r = build_records(L, l, p, h->bounds, P.mgparam, P.mgform, P.icnd, true, false);
-      ok = ok && r.pos == sor[p].pos;
-      for (uint32_t z : r.zero) ok = ok && z == 0;
+    const Level &Lc = *h->lv[l + 1];
+    if (L.legdown.made < 0) {
+      L.legdown.made = make_tiles(h, L, Lc, L.legdown, false);
+      L.legup.made = L.legdown.made && make_tiles(h, L, Lc, L.legup, true);
     }
-    ok = ok && !(faces_of(h, L) & (FACES_NO | FACES_UNEVEN));
-    L.legcls.release();
+    bool ok = L.legdown.made && L.legup.made && !(faces_of(h, L) & (FACES_NO | FACES_UNEVEN));
+    if (L.hasmask) {
+      // (the same points are active in the sweeps and in the residual)
+      const CondDev<double> &C = cond_of<double>(L);
+      for (int p = 0; p < 2; p++)
+        ok = ok && C.res[0][p].n == (int)L.rec_h[p].size() / 3 && !C.res[0][p].anyzero;
+    }
     if (ok && L.hasmask) {
       std::vector<uint8_t> cls((size_t)(2 * L.g.cs), (uint8_t)LEG_DENSE);
-      if (L.nint > 0) {
-        std::vector<int> hp(3 * L.nint);
-        WM_HIP(hipMemcpy(hp.data(), L.int_pos.p, sizeof(int) * hp.size(), hipMemcpyDeviceToHost));
-        for (int i = 0; i < L.nint; i++)
-          cls[rb_index(L.g, hp[3 * i], hp[3 * i + 1], hp[3 * i + 2])] = LEG_INT;
-      }
-      for (int p = 0; p < 2; p++)
-        for (int i = 0; i < sor[p].n(); i++)
-          cls[rb_index(L.g, sor[p].pos[3 * i], sor[p].pos[3 * i + 1], sor[p].pos[3 * i + 2])] =
-              LEG_REC;
+      for (size_t i = 0; i + 2 < L.int_h.size(); i += 3)
+        cls[rb_index(L.g, L.int_h[i], L.int_h[i + 1], L.int_h[i + 2])] = LEG_INT;
+      for (const std::vector<int> &q : L.rec_h)
+        for (size_t i = 0; i + 2 < q.size(); i += 3)
+          cls[rb_index(L.g, q[i], q[i + 1], q[i + 2])] = LEG_REC;
       // the sides across which a point reads an interior one before its pin
       for (size_t e = 0; e < L.raw_h.size(); e++)
         if (cls[e] != LEG_INT) cls[e] |= (uint8_t)(L.raw_h[e] << 2);
       L.legcls.upload(cls);
     }
-    const Level &Lc = *h->lv[l + 1];
-    ok = ok && build_leg(h, L, Lc, L.legdown, false, sor) && build_leg(h, L, Lc, L.legup, true, sor);
-    if (ok != L.leg_ok || ok) {
-      h->drop_graphs();  // captured V-cycles hold the old tables' addresses
+    if (ok) {
+      place_records(L, L.legdown);
+      place_records(L, L.legup);
+      h->drop_graphs();  // captured V-cycles may hold other tables' addresses
       h->gkey = wm_mg3d::GKey();
     }
     L.leg_ok = ok;
@@ -2266,8 +2283,8 @@ static LegArgs<S> leg_args(wm_mg3d *h, Level &L, const Level &Lc, const LegTiles
   A.rz = (S)(L.dzsqi * P.mgparam * cr);
   A.mgparam = (S)P.mgparam;
   A.ff = L.ff;
-  A.cls = L.legcls.p;
-  if (P.lcnd && D.rec.p) {
+  A.cls = L.hasmask ? L.legcls.p : nullptr;
+  if (P.lcnd && D.nrec > 0) {
     A.first = D.first.p;
     A.rec = D.rec.p;
     CondDev<S> &C = cond_of<S>(L);
@@ -2668,6 +2685,7 @@ int wm_mg3d_set_conductors(wm_mg3d *h, const wm_conductor_lists *c) {
       L.c64.reset();
       L.c32.reset();
       L.legkey = RecKey();
+      L.int_h.clear();
       L.faces = -1;
       L.raw_h.clear();
     }
@@ -2695,6 +2713,7 @@ int wm_mg3d_set_conductors(wm_mg3d *h, const wm_conductor_lists *c) {
         L.nint = (int)volt.size();
         L.int_pos.upload(pos);
         L.int_volt.upload(volt);
+        if (l > 0) L.int_h.swap(pos);
       }
       for (int p = 0; p < 2; p++) {
         if (c->sub_n[p] == 0) continue;
