@@ -82,7 +82,7 @@ struct LegArgs {
   SubList<T> sor[2], res[2];
 };
 
-enum { LEG_DENSE = 0, LEG_REC = 1, LEG_INT = 2, LEG_OUT = 3 };
+enum { LEG_DENSE = 0, LEG_REC = 1, LEG_INT = 2 };
 constexpr int LEG_TH = 512;  // threads of a block
 constexpr int LEG_NI = 4;    // pairs of points per thread, at most
 // Coarse nodes of a tile along one axis, at most (down); points of a window.
