@@ -564,9 +564,10 @@ struct __attribute__((packed, aligned(8))) Pair {
 // order.  Particles outside the grid get no field.
 //
 // The 32 values are read as 16 pairs along x.  What bounds a gather by
-// particles in no order is the cache lines they touch (12 rows each, from
-// beyond the L2 on a mesh of 35 MB), but fewer loads still help: 1M particles
-// on 128x128x256 83 -> 79 us, the push of 4M ordered ones 113 -> 110 us.
+// particles in no order is the cache lines that they ask the L2 for (12 rows, 14
+// lines each: 22.6 TB/s on a mesh of 35 MB, of which the L2 holds 85%), but
+// fewer loads still help: 1M particles on 128x128x256 83 -> 79 us, the push
+// of 4M ordered ones 113 -> 110 us.
 __device__ inline void gather_e(const double *__restrict__ phi, const Mesh &m, double tdxi,
                                 double tdyi, double tdzi, double x, double y, double z,
                                 double &ext, double &eyt, double &ezt) {
