@@ -574,6 +574,51 @@ def test_coarse_levels_conductors_at_faces(device, case, passes, monkeypatch):
         np.testing.assert_array_equal(a[2], b[2])
 
 
+@pytest.mark.parametrize("precision", ["fp64", "bf16"])
+def test_solve_after_level_calls_with_other_settings(device, precision):
+    """Between two solves of one setting, a residual, a half sweep and a pass
+    of single levels with others, which upload other records: the second solve
+    runs on its own records, with the bits of a solver that made the two
+    solves alone."""
+    import warp_amd
+    from warp_amd import _native as N
+    from warp_amd import configs
+    n = (64, 48, 96)
+    rng = np.random.default_rng(3)
+    rho = torch.from_numpy(1e-4 * rng.normal(size=(n[2] + 1, n[1] + 1, n[0] + 1))).to(device)
+    out = []
+    for between in (False, True):
+        s = _solver(*n, (-0.02, -0.02, 0.0), (0.02, 0.02, 0.08), (0,) * 6, precision=precision,
+                    mgmaxiters=8)
+        for g in configs.conductors("pipe_annulus", warp_amd):
+            s.installconductor(g)
+        s.rho = rho
+        s.solve()
+        assert s.leg_levels()
+        if between:
+            s.lcndbndy = False
+            s.getresidual()
+            s.lcndbndy = True
+            for level, icnd in ((0, 1), (1, 1), (1, 2), (2, 1)):
+                d = (C.c_int64 * 3)()
+                N.call("wm_mg3d_level_dims", s._h, level, d, None)
+                phi = torch.zeros((d[2] + 3, d[1] + 3, d[0] + 3), dtype=torch.float64,
+                                  device=device)
+                r = torch.zeros((d[2] + 1, d[1] + 1, d[0] + 1), dtype=torch.float64,
+                                device=device)
+                for lcnd in (0, 1):
+                    N.call("wm_mg3d_sorpass", s._h, level, phi.data_ptr(), r.data_ptr(), 1.6, 1,
+                           lcnd, icnd, N.stream_of(device))
+                    N.call("wm_mg3d_sorhalfpass", s._h, level, 1, phi.data_ptr(), r.data_ptr(),
+                           1.6, 1, lcnd, icnd, N.stream_of(device))
+            torch.cuda.synchronize()
+        s.rho = 1.1 * rho
+        s.solve()
+        out.append((s.mgiters, s.mgerror, s.phi.cpu().numpy().copy()))
+    assert out[0][:2] == out[1][:2]
+    np.testing.assert_array_equal(out[0][2], out[1][2])
+
+
 @pytest.mark.parametrize("bounds", [(0,) * 6, (1, 1, 0, 1, 2, 2), (2, 2, 1, 0, 0, 1)])
 def test_residual_wide_rows_match_oracle(device, bounds):
     """residual3d on a level with padded rows (nx = 128: 80 elements per

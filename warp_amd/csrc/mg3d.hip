@@ -141,7 +141,9 @@ struct SubDev {
   DevBuf<T> k, denom, fac;
   int n = 0;
   bool anyzero = false;  // some record zeroes a neighbour's residual
-  void upload(const SubHost &h) {
+  // Returns whether an array has moved.
+  bool upload(const SubHost &h) {
+    const void *was[6] = {pos.p, modes.p, zero.p, k.p, denom.p, fac.p};
     n = h.n();
     anyzero = false;
     for (uint32_t z : h.zero) anyzero = anyzero || z != 0;
@@ -153,6 +155,8 @@ struct SubDev {
     k.upload(kk);
     denom.upload(dd);
     fac.upload(ff);
+    const void *is[6] = {pos.p, modes.p, zero.p, k.p, denom.p, fac.p};
+    return !std::equal(was, was + 6, is);
   }
   SubList<T> view() const {
     return SubList<T>{n, pos.p, modes.p, k.p, denom.p, fac.p, zero.p};
@@ -329,6 +333,10 @@ struct wm_mg3d {
              mgtol == o.mgtol;
     }
   } gkey;
+  void forget_graphs() {
+    drop_graphs();
+    gkey = GKey();
+  }
   int last_iters = 0;
   // SOR pass form: 0 two half sweeps, 1 the fused two-colour pass where it
   // applies, 2 the fused pass on the finest level only
@@ -687,8 +695,8 @@ static void build_mask(wm_mg3d *h, Level &L, int level, const Params &P) {
     long long e = rb_index(L.g, ix, iy, iz);
     m[e >> 5] |= 1u << (e & 31);
   };
-  std::vector<int> ipos;
   bool any = false;
+  const uint32_t *was[2] = {L.mask.p, L.imask.p};
   if (L.nint > 0) {
     std::vector<int> down;
     if (level == 0) {
@@ -720,10 +728,14 @@ static void build_mask(wm_mg3d *h, Level &L, int level, const Params &P) {
   }
   if (any) L.mask.upload(m);
   else L.mask.release();
+  if (L.mask.p != was[0] || L.imask.p != was[1]) h->forget_graphs();
   L.hasmask = any;
   L.maskkey = key;
 }
 
+// Here and in build_mask: captured V-cycles hold these arrays' addresses, and
+// the entry points of single levels may ask for another setting's between two
+// solves of one, so the graphs go where an array moves.
 template <typename T>
 static void ensure_records(wm_mg3d *h, Level &L, int level, const Params &P,
                            bool residual, int mgform2init) {
@@ -741,7 +753,7 @@ static void ensure_records(wm_mg3d *h, Level &L, int level, const Params &P,
     for (int p = 0; p < 2; p++) {
       SubHost sh;
       if (P.lcnd) sh = build_records(L, level, p, h->bounds, P.mgparam, P.mgform, P.icnd, false, false);
-      C.sor[p].upload(sh);
+      if (C.sor[p].upload(sh)) h->forget_graphs();
     }
     C.sorkey = key;
   } else {
@@ -757,12 +769,14 @@ static void ensure_records(wm_mg3d *h, Level &L, int level, const Params &P,
                                                        (long long)(L.ny + 3) * (sh.pos[3 * i + 2] + 1));
         ord.push_back({nat, ((uint32_t)p << 31) | (uint32_t)i});
       }
-      C.res[mgform2init][p].upload(sh);
+      if (C.res[mgform2init][p].upload(sh)) h->forget_graphs();
     }
     std::sort(ord.begin(), ord.end());
     std::vector<uint32_t> o(ord.size());
     for (size_t i = 0; i < ord.size(); i++) o[i] = ord[i].second;
+    const uint32_t *was = C.resord[mgform2init].p;
     C.resord[mgform2init].upload(o);
+    if (C.resord[mgform2init].p != was) h->forget_graphs();
     C.reskey[mgform2init] = key;
   }
 }
@@ -1952,8 +1966,7 @@ static void prepare_tail(wm_mg3d *h, const Params &P) {
          std::memcmp(h->tail.items.data(), items.data(), sizeof(TailItem) * items.size()) == 0);
     if (!same) {
       // captured V-cycles hold the old step count and sizes by value
-      h->drop_graphs();
-      h->gkey = wm_mg3d::GKey();
+      h->forget_graphs();
       WM_HIP(hipStreamSynchronize(h->s));
       WM_HIP(hipMemset(h->tailimage.p, 0, sizeof(uint32_t) * h->tailimage.n));
       WM_HIP(hipMemcpy(h->taildesc.p, desc.data(), desc.size(), hipMemcpyHostToDevice));
@@ -2246,8 +2259,7 @@ static void prepare_legs(wm_mg3d *h, const Params &P) {
     if (ok) {
       place_records(L, L.legdown);
       place_records(L, L.legup);
-      h->drop_graphs();  // captured V-cycles may hold other tables' addresses
-      h->gkey = wm_mg3d::GKey();
+      h->forget_graphs();  // captured V-cycles may hold other tables' addresses
     }
     L.leg_ok = ok;
   }
@@ -2691,8 +2703,7 @@ int wm_mg3d_set_conductors(wm_mg3d *h, const wm_conductor_lists *c) {
     }
     h->conductors_set = false;
     h->last_ok = false;
-    h->drop_graphs();
-    h->gkey = wm_mg3d::GKey();
+    h->forget_graphs();
     if (c == nullptr) return 0;
     WM_REQUIRE(c->levels >= (int64_t)h->lv.size() || (c->int_n == 0 && c->sub_n[0] == 0 && c->sub_n[1] == 0),
                "wm_mg3d_set_conductors: conductor data has fewer levels than the solver");
@@ -2865,8 +2876,7 @@ int wm_mg3d_solve(wm_mg3d *h, double *phi, double *rho, double mgparam, int64_t 
       if (P.lcnd) nrec = cond_of<double>(L0).sor[0].n + cond_of<double>(L0).sor[1].n;
       long long cap = 2 * ((long long)(g0.W / 64 + 1) * (g0.PY + 16) * g0.PZ) + nrec / 64 + 4096;
       if ((long long)h->convparts.n < cap) {
-        h->drop_graphs();  // captured graphs hold the old buffer's address
-        h->gkey = wm_mg3d::GKey();
+        h->forget_graphs();  // captured graphs hold the old buffer's address
         h->convparts.alloc((size_t)cap);
       }
     }
@@ -3073,8 +3083,7 @@ int wm_mg3d_set_sor_form(wm_mg3d *h, int64_t form) {
     WM_REQUIRE(h != nullptr, "wm_mg3d_set_sor_form: NULL handle");
     WM_REQUIRE(form >= 0 && form <= 2, "wm_mg3d_set_sor_form: form must be 0, 1 or 2");
     if (h->sor_form != (int)form) {
-      h->drop_graphs();  // captured V-cycles hold the other form's launches
-      h->gkey = wm_mg3d::GKey();
+      h->forget_graphs();  // captured V-cycles hold the other form's launches
       h->last_ok = false;
       h->sor_form = (int)form;
     }
