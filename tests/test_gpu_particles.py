@@ -169,6 +169,42 @@ def test_deposits_on_two_streams(device, grow):
     assert np.abs(s.rho.cpu().numpy() - ro).max() <= 1e-13 * np.abs(ro).max()
 
 
+def test_deposit_captured(device):
+    """A deposit captured into a graph (its workspace from the graph's pool)
+    and replayed, with eager deposits of another count between: rho as the
+    oracle sums it, 1e-13 of the peak."""
+    from warp_amd.multigrid import MultiGrid3D
+    s = MultiGrid3D(nx=NX, ny=NY, nz=NZ, xmmin=LO[0], xmmax=-LO[0], ymmin=LO[1], ymmax=-LO[1],
+                    zmmin=LO[2], zmmax=LO[2] + NZ * DZ, bounds=[0] * 6, device=device,
+                    mgverbose=-1)
+    beams = [_beam(300000, 3), _beam(120000, 4)]
+    ro = []
+    for b in beams:
+        r = np.zeros((NZ + 1, NY + 1, NX + 1))
+        O.setrho3d(r, *b, 1., 2., s.dx, s.dy, s.dz, *LO)
+        ro.append(r)
+    dev = [[_t(v, device) for v in b] for b in beams]
+
+    def deposit(i):
+        s.zerosourcep()
+        s.setsourcepatposition(*dev[i], 0., 1., 2.)
+
+    def right(i):
+        torch.cuda.synchronize()
+        return np.abs(s.rho.cpu().numpy() - ro[i]).max() <= 1e-13 * np.abs(ro[i]).max()
+
+    deposit(0)
+    assert right(0)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        deposit(0)
+    for _ in range(3):
+        g.replay()
+        assert right(0)
+        deposit(1)
+        assert right(1)
+
+
 def test_deposit_where_the_workspace_does_not_fit(device, monkeypatch):
     """No memory for the workspace: the deposit does without it."""
     from warp_amd.multigrid import MultiGrid3D

@@ -407,3 +407,18 @@ def test_few_unordered_particles_are_binned():
     v = torch.zeros(3, dtype=torch.float64)
     pg.addparticles(0, *[v] * 6)
     assert not pg.ordered
+
+
+def test_deposit_workspace_of_the_wrong_kind_is_refused():
+    """Too small, or not aligned: an error from the host, before any launch."""
+    import ctypes as C
+    from warp_amd import _native as N
+    mesh = (64, 64, 64)
+    need = N.lib().wm_setrho3d_worksize(40000, *mesh)
+    assert need > 0
+    # (addresses that nothing reads)
+    for work, size, what in ((4096, need - 1, "too small"), (4097, need, "not aligned"),
+                             (4100, need, "not aligned")):
+        rc = N.lib().wm_setrho3d_work(4096, 40000, 4096, 4096, 4096, 0., 1., 1., *mesh, 1., 1., 1.,
+                                      0., 0., 0., None, C.c_void_p(work), size, None)
+        assert rc != 0 and what in N.lib().wm_last_error().decode()

@@ -1071,6 +1071,8 @@ int wm_setrho3d_work(double *rho, int64_t np, const double *xp, const double *yp
     WM_REQUIRE(rho && xp && yp && zp, "wm_setrho3d: NULL array");
     const BinLayout w = work ? bin_layout(np, nx, ny, nz) : BinLayout{};
     WM_REQUIRE(!w.total || worksize >= (int64_t)w.total, "wm_setrho3d: workspace too small");
+    // (its counters are updated by atomics, which fault on a split word)
+    WM_REQUIRE(!w.total || ((uintptr_t)work & 7) == 0, "wm_setrho3d: workspace not aligned");
     hipStream_t s = wm_stream(stream);
     Mesh m = make_mesh(nx, ny, nz, dx, dy, dz, xmmin, ymmin, zmmin, zgrid);
     double g = deposit_g(q, wght, nx, ny, nz, dx, dy, dz);
