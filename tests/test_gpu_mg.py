@@ -529,11 +529,17 @@ def test_vcycle_legs_same_bits(device, case, precision, monkeypatch):
 
 
 @pytest.mark.parametrize("case", [
-    # mesh, bounds: interior points beside faces on some levels and on them on
-    # others, on one plane of a periodic axis alone, levels that halve and not
-    ((32, 32, 64), (0, 0, 0, 0, 2, 2)), ((32, 48, 32), (1, 1, 1, 0, 0, 1)),
-    ((64, 32, 32), (2, 2, 1, 1, 2, 2)), ((40, 24, 56), (1, 0, 2, 2, 0, 0)),
-    ((33, 37, 48), (0, 1, 1, 1, 2, 2))])
+    # mesh, bounds, a conductor across the high faces of x and y or beside them,
+    # legs: interior points beside faces on some levels and on them on others, on
+    # one plane of a periodic axis alone (no legs then), levels that halve and not
+    ((32, 32, 64), (0, 0, 0, 0, 2, 2), True, True),
+    ((32, 48, 32), (1, 1, 1, 0, 0, 1), True, True),
+    ((64, 32, 32), (2, 2, 1, 1, 2, 2), True, False),
+    ((40, 24, 56), (1, 0, 2, 2, 0, 0), True, False),
+    ((33, 37, 48), (0, 1, 1, 1, 2, 2), True, True),
+    ((64, 32, 32), (2, 2, 1, 1, 2, 2), False, True),
+    ((40, 24, 56), (1, 0, 2, 2, 0, 0), False, True),
+    ((36, 42, 40), (2, 2, 2, 2, 1, 0), False, True)])
 @pytest.mark.parametrize("passes", [(1, 1), (2, 2), (1, 0)])
 def test_coarse_levels_conductors_at_faces(device, case, passes, monkeypatch):
     """Coarse levels in one launch each and in the tail's single launch, where
@@ -541,10 +547,11 @@ def test_coarse_levels_conductors_at_faces(device, case, passes, monkeypatch):
     the launches step by step (with their boundary conditions and pins), with
     conductors that touch, nearly touch and cross the faces: the same bits."""
     import warp_amd
-    (nx, ny, nz), bounds = case
+    (nx, ny, nz), bounds, across, legs = case
     rng = np.random.default_rng(9)
     rho = 1e-4 * rng.normal(size=(nz + 1, ny + 1, nx + 1))
-    dx, dz = 0.04 / nx, 0.08 / nz
+    dx, dy, dz = 0.04 / nx, 0.04 / ny, 0.08 / nz
+    corner = (0.0165, 0.016) if across else (0.015 - 1.3 * dx, 0.015 - 0.8 * dy)
     out = []
     for off in (True, False):
         for k in ("WARPMI_LEG_NODES", "WARPMI_TAIL_LDS"):
@@ -557,7 +564,7 @@ def test_coarse_levels_conductors_at_faces(device, case, passes, monkeypatch):
                 (0.006, 0.020, (0.0, 0.0, 0.010 + 1.3 * dz), 50.),            # above z low
                 (0.005, 0.012, (0.009, 0.0, 0.074 - 0.7 * dz), -20.),         # below z high
                 (0.004, 0.030, (-0.016 + 1.6 * dx, -0.012, 0.04), 10.),       # beside x low
-                (0.005, 0.014, (0.0165, 0.016, 0.045), 5.)):                  # across x, y high
+                (0.005, 0.014, (*corner, 0.045), 5.)):                        # at x, y high
             s.installconductor(warp_amd.ZCylinder(r, length, voltage=v, xcent=at[0], ycent=at[1],
                                                   zcent=at[2]))
         s.downpasses, s.uppasses = passes
@@ -566,7 +573,7 @@ def test_coarse_levels_conductors_at_faces(device, case, passes, monkeypatch):
             s.rho = torch.from_numpy(rho * f).to(device)
             s.solve()
             res.append((s.mgiters, s.mgerror, s.phi.cpu().numpy().copy()))
-            assert not s.leg_levels() or (not off and passes == (1, 1))
+            assert bool(s.leg_levels()) == (legs and not off and passes == (1, 1))
         out.append(res)
         assert (s.tail_start_level() > 0) != off
     for a, b in zip(*out):
